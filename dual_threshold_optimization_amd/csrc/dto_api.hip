@@ -145,6 +145,11 @@ int prepare_job(dto_job *j) {
                                        std::to_string(lim));
   j->lo_plain = without_h;
   j->lo_screen = screen_layout(h, kNT / 64, lim);
+  const HostJob *hp = &h;
+  if ((rc = cut_shape(&hp, 1, lim, &j->cut_sh))) return rc;
+  (void)cut_layout(h, j->cut_sh.nt / 64, j->cut_sh.build, &j->lo_cut);
+  if (j->cut) (void)hipFree(j->cut);
+  j->cut = nullptr;
   std::vector<unsigned char> &buf = j->image;
   buf.clear();
   ArenaOffsets &o = j->off;
@@ -179,6 +184,7 @@ int prepare_job(dto_job *j) {
   d.dup = h.dup ? 1u : 0u;
   d.kle = h.kle ? 1u : 0u;
   d.margin = h.margin;
+  cut_levels(h, d);
   return DTO_OK;
 }
 
@@ -224,20 +230,12 @@ int upload_job(dto_job *j) {
     (void)hipFree(j->ws);
     j->ws = nullptr;
   }
-  if (j->gnb) {
-    (void)hipFree(j->gnb);
-    j->gnb = nullptr;
-  }
   j->ws_slots = (uint32_t)pr.cus * 4u;
-  if (!j->lo_plain.pairs_in_lds || !j->lo_screen.pairs_in_lds) {
+  if (!j->lo_plain.pairs_in_lds || !j->lo_cut.pairs_in_lds) {
     HIP_TRY(hipMalloc(&j->ws, (size_t)j->ws_slots * std::max<uint32_t>(j->dev.N2, 1) * sizeof(uint16_t)));
     if (!j->ws_ev) HIP_TRY(hipEventCreateWithFlags(&j->ws_ev, hipEventDisableTiming));
   }
-  if (!j->lo_screen.nb_in_lds) {
-    HIP_TRY(hipMalloc(&j->gnb, (size_t)j->ws_slots * std::max(std::max(j->dev.N1, j->dev.N2), 1u) * sizeof(uint16_t)));
-    if (!j->ws_ev) HIP_TRY(hipEventCreateWithFlags(&j->ws_ev, hipEventDisableTiming));
-  }
-  return DTO_OK;
+  return ensure_cut(j, 0);
 }
 
 int ensure_resident(dto_job *j) {
@@ -248,103 +246,56 @@ int ensure_resident(dto_job *j) {
 /* ------------------------------------------------------------------ */
 /* launches                                                              */
 /* ------------------------------------------------------------------ */
-/* Launches that stage their pairs or keep their bins in the job's global
- * buffers (lists too long for the LDS) run one after another, whatever their
- * streams: each waits for the previous one's completion event.  Inside a stream capture the wait is
- * left out (a capture cannot wait on work recorded outside it), so captured
- * launches of one such job must not overlap. */
-struct StagingOrder {
-  dto_job *j;
-  hipStream_t st;
-  bool on = false;
-  StagingOrder(const dto_job *job, const LdsLayout &lo, hipStream_t s) : j(const_cast<dto_job *>(job)), st(s) {
-    if ((lo.pairs_in_lds && lo.nb_in_lds) || !j->ws_ev) return;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
-    if (cs != hipStreamCaptureStatusNone) return;
-    j->ws_mu.lock();
-    on = true;
-    if (j->ws_used) (void)hipStreamWaitEvent(st, j->ws_ev, 0);
-  }
-  ~StagingOrder() {
-    if (!on) return;
-    if (hipEventRecord(j->ws_ev, st) == hipSuccess) j->ws_used = true;
-    j->ws_mu.unlock();
-  }
-};
-
-template <bool E, bool HL, bool PL, bool PA, bool RC, bool NBL = true>
+/* The plain kernel (every cell exact). */
+template <bool E, bool PA>
 static hipError_t launch_opt(const dto_job *j, const LdsLayout &lo, uint32_t grid, hipStream_t st,
                              const uint32_t *i1, const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed,
                              uint32_t job_id, int32_t permuted, dto_record *out) {
-  auto kern = k_optimize<kNT, E, HL, PL, PA, RC, NBL>;
+  auto kern = k_optimize<kNT, E, false, true, PA, false, true>;
   (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lo.total);
   /* a slot of the job's counter ring for this launch, zeroed on its stream */
   uint32_t *ctr = j->d_ctr + (const_cast<dto_job *>(j)->ctr_next.fetch_add(1u) % kCounterRing);
   StagingOrder order(j, lo, st);
   hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, ctr);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kNT), lo.total, st, j->dev, lo, i1, i2, n_perm, base, seed, job_id,
-                     permuted, out, j->d_err, j->ws, j->gnb, ctr);
+                     permuted, out, j->d_err, j->ws, nullptr, ctr);
   return hipGetLastError();
-}
-
-/* Lane segments fit in registers when a row is at most kSegWords words per lane. */
-static bool regcols(const dto_job *j) { return (j->dev.T2w + 63) / 64 <= kSegWords; }
-
-template <bool E, bool HL, bool PL>
-static hipError_t launch_opt_r(const dto_job *j, const LdsLayout &lo, uint32_t grid, hipStream_t st,
-                               const uint32_t *i1, const uint32_t *i2, uint64_t n_perm, uint64_t base,
-                               uint64_t seed, uint32_t job_id, int32_t permuted, dto_record *out) {
-  if (PL) /* the plain kernel reads column constants per cell; one variant */
-    return lo.pairs_in_lds
-               ? launch_opt<E, false, true, true, false>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out)
-               : launch_opt<E, false, true, false, false>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
-  const bool rc = regcols(j);
-  if (HL && !lo.nb_in_lds) /* the table in LDS, the bins global (pairs alias the table) */
-    return rc ? launch_opt<E, true, false, true, true, false>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id,
-                                                              permuted, out)
-              : launch_opt<E, true, false, true, false, false>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id,
-                                                               permuted, out);
-  if (lo.pairs_in_lds) {
-    if (rc) return launch_opt<E, HL, false, true, true>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
-    return launch_opt<E, HL, false, true, false>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
-  }
-  if (rc) return launch_opt<E, false, false, false, true>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
-  return launch_opt<E, false, false, false, false>(j, lo, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
 }
 
 /* Number of workgroups for a permutation launch: enough to fill every CU at
  * the occupancy the LDS footprint allows, never more than the work. */
-static uint32_t perm_grid(const dto_job *j, const LdsLayout &lo, uint64_t n_perm) {
+static uint32_t perm_grid(const dto_job *j, const LdsLayout &lo, uint64_t n_perm, uint64_t max_per_cu) {
   DevProps pr;
   if (device_props(j->device, &pr)) return 1;
   uint64_t per_cu = std::max<uint64_t>(1, pr.lds_per_block ? (160u * 1024u) / std::max<uint32_t>(lo.total, 1) : 1);
-  per_cu = std::min<uint64_t>(per_cu, 4);
+  per_cu = std::min<uint64_t>(per_cu, max_per_cu);
   uint64_t g = std::min<uint64_t>(n_perm, (uint64_t)pr.cus * per_cu);
-  if (!lo.pairs_in_lds || !lo.nb_in_lds) g = std::min<uint64_t>(g, j->ws_slots); /* one global slot per workgroup */
+  if (!lo.pairs_in_lds) g = std::min<uint64_t>(g, j->ws_slots); /* one global slot per workgroup */
   return (uint32_t)std::max<uint64_t>(g, 1);
 }
 
+/* lead = 1: the unpermuted task runs first, in the same launch, into record 0
+ * (screened mode with drawn permutations only). */
 static int launch_perms(dto_job *j, uint32_t mode, bool expl, const uint32_t *d1, const uint32_t *d2, uint64_t n_perm,
                         uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted, dto_record *d_out,
-                        hipStream_t st) {
-  if (n_perm == 0) return DTO_OK;
+                        hipStream_t st, uint32_t lead = 0) {
+  if (n_perm + lead == 0) return DTO_OK;
   if (n_perm >= (1ull << 32) - 65536ull) return fail(DTO_ERR_TOO_LARGE, "too many permutations in one launch");
   hipError_t e;
   if (mode == DTO_MODE_PLAIN) {
     const LdsLayout &lo = j->lo_plain;
-    uint32_t g = perm_grid(j, lo, n_perm);
-    e = expl ? launch_opt_r<true, false, true>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
-             : launch_opt_r<false, false, true>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
-  } else if (mode == DTO_MODE_SCREENED) {
-    const LdsLayout &lo = j->lo_screen;
-    uint32_t g = perm_grid(j, lo, n_perm);
-    if (lo.h_in_lds)
-      e = expl ? launch_opt_r<true, true, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
-               : launch_opt_r<false, true, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
+    const uint32_t g = perm_grid(j, lo, n_perm, 4);
+    if (expl)
+      e = lo.pairs_in_lds ? launch_opt<true, true>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
+                          : launch_opt<true, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
     else
-      e = expl ? launch_opt_r<true, false, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
-               : launch_opt_r<false, false, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
+      e = lo.pairs_in_lds ? launch_opt<false, true>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
+                          : launch_opt<false, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
+  } else if (mode == DTO_MODE_SCREENED) {
+    int rc = ensure_cut(j, st);
+    if (rc) return rc;
+    const uint32_t g = perm_grid(j, j->lo_cut, n_perm + lead, j->cut_sh.nt == 512 ? 4 : 2);
+    e = launch_cut(j, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, lead, d_out);
   } else {
     return fail(DTO_ERR_INVALID_ARGUMENT, "unknown mode");
   }
@@ -661,7 +612,7 @@ void dto_job_destroy(dto_job *job) {
   if (!job) return;
   if (job->arena) (void)hipFree(job->arena);
   if (job->ws) (void)hipFree(job->ws);
-  if (job->gnb) (void)hipFree(job->gnb);
+  if (job->cut) (void)hipFree(job->cut);
   if (job->ws_ev) (void)hipEventDestroy(job->ws_ev);
   delete job;
 }
@@ -750,8 +701,10 @@ int dto_run(dto_job *job, uint64_t n_perm, uint64_t seed, const uint32_t *idx1, 
   DevBuf dr;
   HIP_TRY(hipMalloc(&dr.p, (n_perm + 1) * sizeof(dto_record)));
   dto_record *d_rec = (dto_record *)dr.p;
-  /* task 0: unpermuted (main.rs:122-125) */
-  if ((rc = launch_perms(job, mode, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_rec, 0))) return rc;
+  /* task 0: unpermuted (main.rs:122-125); with drawn permutations it joins
+   * their launch, where it costs no workgroup's latency of its own */
+  const uint32_t lead = mode == DTO_MODE_SCREENED && n_perm && !idx1 ? 1 : 0;
+  if (!lead && (rc = launch_perms(job, mode, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_rec, 0))) return rc;
   if (n_perm) {
     if (idx1) {
       /* explicit permutations, streamed in chunks of at most ~512 MiB */
@@ -768,7 +721,8 @@ int dto_run(dto_job *job, uint64_t n_perm, uint64_t seed, const uint32_t *idx1, 
         HIP_TRY(hipDeviceSynchronize());
       }
     } else {
-      if ((rc = launch_perms(job, mode, false, nullptr, nullptr, n_perm, 0, seed, 0, 1, d_rec + 1, 0))) return rc;
+      if ((rc = launch_perms(job, mode, false, nullptr, nullptr, n_perm, 0, seed, 0, 1, d_rec + 1 - lead, 0, lead)))
+        return rc;
     }
   }
   std::vector<dto_record> rec(n_perm + 1);

@@ -37,8 +37,8 @@ using namespace dto;
 
 namespace {
 
-/* Launch shapes the batch kernels are built for: threads per workgroup, the
- * screen table in LDS or not, the pair staging in LDS or global memory. */
+/* Launch shapes of a server's slices: the screen table in LDS or not, the
+ * bins and the pair staging in LDS or global memory. */
 /* Global buffers of a launch: pair staging (ws, ws_stride u16 per
  * workgroup) and bins arrays (gnb, gnb_stride u16 per workgroup). */
 struct Globals {
@@ -47,7 +47,7 @@ struct Globals {
 };
 
 template <int NT, bool HL, bool PL, bool RC, bool NBL>
-hipError_t launch_batch_t(uint32_t grid, uint32_t lds, hipStream_t st, const BatchJob *jobs, const WorkItem *items,
+hipError_t launch_slice_t(uint32_t grid, uint32_t lds, hipStream_t st, const BatchJob *jobs, const WorkItem *items,
                           uint32_t n_items, uint64_t seed, uint32_t *counter, int *err, const Globals &g) {
   auto kern = k_batch<NT, HL, PL, RC, NBL>;
   (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -57,75 +57,42 @@ hipError_t launch_batch_t(uint32_t grid, uint32_t lds, hipStream_t st, const Bat
   return hipGetLastError();
 }
 
-template <int NT>
-hipError_t launch_batch_n(bool hl, bool nbl, bool pl, bool rc, uint32_t grid, uint32_t lds, hipStream_t st,
+hipError_t launch_slice(bool hl, bool nbl, bool pl, bool rc, uint32_t grid, uint32_t lds, hipStream_t st,
                           const BatchJob *jobs, const WorkItem *items, uint32_t n_items, uint64_t seed,
                           uint32_t *counter, int *err, const Globals &g) {
   if (hl && nbl)
-    return rc ? launch_batch_t<NT, true, true, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
-              : launch_batch_t<NT, true, true, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
+    return rc ? launch_slice_t<kNT, true, true, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
+              : launch_slice_t<kNT, true, true, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
   if (hl)
-    return rc ? launch_batch_t<NT, true, true, true, false>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
-              : launch_batch_t<NT, true, true, false, false>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
+    return rc ? launch_slice_t<kNT, true, true, true, false>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
+              : launch_slice_t<kNT, true, true, false, false>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
   if (pl)
-    return rc ? launch_batch_t<NT, false, true, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
-              : launch_batch_t<NT, false, true, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
-  return rc ? launch_batch_t<NT, false, false, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
-            : launch_batch_t<NT, false, false, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
+    return rc ? launch_slice_t<kNT, false, true, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
+              : launch_slice_t<kNT, false, true, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
+  return rc ? launch_slice_t<kNT, false, false, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
+            : launch_slice_t<kNT, false, false, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
 }
 
-/* Batch-wide launch parameters for a set of jobs at nt threads. */
+/* One launch shape for all jobs of a batch, with each job's layout. */
 struct Shape {
-  int nt = 512;
-  bool hl = true;  /* screen table in LDS */
-  bool nbl = true; /* bins arrays in LDS */
-  bool pl = true;  /* pair staging in LDS */
-  bool rc = true;  /* every job's lane segment fits in registers */
-  uint32_t lds = 0;
-  uint32_t max_n2 = 0, max_n = 0; /* largest N2, largest max(N1, N2) */
+  CutShape cut;
+  uint32_t max_n2 = 0; /* largest N2 */
   std::vector<LdsLayout> lo;
 };
 
-hipError_t launch_batch(const Shape &sh, uint32_t grid, hipStream_t st, const BatchJob *jobs, const WorkItem *items,
-                        uint32_t n_items, uint64_t seed, uint32_t *counter, int *err, const Globals &g) {
-  hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, st, counter, err);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (sh.nt == 256)
-    return launch_batch_n<256>(sh.hl, sh.nbl, sh.pl, sh.rc, grid, sh.lds, st, jobs, items, n_items, seed, counter,
-                               err, g);
-  return launch_batch_n<512>(sh.hl, sh.nbl, sh.pl, sh.rc, grid, sh.lds, st, jobs, items, n_items, seed, counter, err,
-                             g);
-}
-
-/* One shape for all jobs of a launch: the first of (table and bins in
- * LDS), (table in LDS, bins global), (table global) that every job fits. */
-int plan_shape(const std::vector<dto_job *> &jobs, int nt, size_t lds_limit, Shape &s) {
-  s.nt = nt;
-  const int W = nt / 64;
-  bool fit_hb = true, fit_h = true, fit_p = true;
+int plan_shape(const std::vector<dto_job *> &jobs, size_t lds_limit, Shape &s) {
+  std::vector<const HostJob *> hs;
+  for (dto_job *j : jobs) hs.push_back(&j->h);
+  int rc = cut_shape(hs.data(), hs.size(), lds_limit, &s.cut);
+  if (rc) return rc;
   s.max_n2 = 1;
-  s.max_n = 1;
-  s.rc = true;
-  for (dto_job *j : jobs) {
-    if ((j->dev.T2w + 63) / 64 > kSegWords) s.rc = false;
-    if (make_layout(j->h, W, true, lds_limit, true).total > lds_limit) fit_hb = false;
-    if (make_layout(j->h, W, true, lds_limit, false).total > lds_limit) fit_h = false;
-    s.max_n2 = std::max(s.max_n2, j->dev.N2);
-    s.max_n = std::max(s.max_n, std::max(j->dev.N1, j->dev.N2));
-  }
-  s.hl = fit_h;
-  s.nbl = fit_hb || !fit_h;
   s.lo.clear();
-  s.lds = 0;
   for (dto_job *j : jobs) {
-    LdsLayout L = make_layout(j->h, W, s.hl, lds_limit, s.nbl);
-    if (L.total > lds_limit) return fail(DTO_ERR_TOO_LARGE, "job does not fit in LDS");
-    if (!L.pairs_in_lds) fit_p = false;
+    LdsLayout L;
+    (void)cut_layout(j->h, s.cut.nt / 64, s.cut.build, &L);
     s.lo.push_back(L);
-    s.lds = std::max(s.lds, L.total);
+    s.max_n2 = std::max(s.max_n2, j->dev.N2);
   }
-  s.pl = fit_p;
   return DTO_OK;
 }
 
@@ -164,8 +131,7 @@ struct dto_batch {
   uint32_t *d_counter = nullptr;
   int *d_err = nullptr;
   dto_record *d_out = nullptr;
-  uint16_t *d_ws = nullptr;  /* global pair staging when the LDS cannot hold the pairs */
-  uint16_t *d_gnb = nullptr; /* global bins arrays when the LDS holds the table but not the bins */
+  uint16_t *d_ws = nullptr; /* global pair staging when the LDS cannot hold the pairs */
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
   hipStream_t own_stream = nullptr;
@@ -179,26 +145,24 @@ static void batch_free_plan(dto_batch *b) {
   if (b->d_jobs) (void)hipFree(b->d_jobs);
   if (b->d_items) (void)hipFree(b->d_items);
   if (b->d_ws) (void)hipFree(b->d_ws);
-  if (b->d_gnb) (void)hipFree(b->d_gnb);
   b->d_jobs = nullptr;
   b->d_items = nullptr;
   b->d_ws = nullptr;
-  b->d_gnb = nullptr;
 }
 
-static Globals batch_globals(const dto_batch *b) {
-  Globals g;
-  g.ws = b->d_ws;
-  g.ws_stride = b->shape.max_n2;
-  g.gnb = b->d_gnb;
-  g.gnb_stride = b->shape.max_n;
-  return g;
+/* Queue reset, then the persistent kernel. */
+static hipError_t batch_kernels(const dto_batch *b, hipStream_t st) {
+  hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, st, b->d_counter, b->d_err);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_batch_cut(b->shape.cut, b->grid, st, b->d_jobs, b->d_items, b->n_items, b->seed, b->d_counter,
+                          b->d_err, b->d_ws, b->shape.max_n2);
 }
 
 /* Builds the job table and the work queue for the current shape and chunk. */
 static int batch_plan(dto_batch *b) {
   batch_free_plan(b);
-  int rc = plan_shape(b->jobs, b->shape.nt, b->lds_limit, b->shape);
+  int rc = plan_shape(b->jobs, b->lds_limit, b->shape);
   if (rc) return rc;
   std::vector<BatchJob> hj(b->jobs.size());
   for (size_t i = 0; i < b->jobs.size(); ++i) {
@@ -232,9 +196,8 @@ static int batch_plan(dto_batch *b) {
   HIP_TRY(hipMalloc(&b->d_items, std::max<size_t>(1, items.size()) * sizeof(WorkItem)));
   HIP_TRY(hipMemcpy(b->d_jobs, hj.data(), hj.size() * sizeof(BatchJob), hipMemcpyHostToDevice));
   if (!items.empty()) HIP_TRY(hipMemcpy(b->d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
-  b->grid = grid_for(b->cus, b->shape.lds, b->shape.nt, b->n_items);
-  if (!b->shape.pl) HIP_TRY(hipMalloc(&b->d_ws, (size_t)b->grid * b->shape.max_n2 * sizeof(uint16_t)));
-  if (!b->shape.nbl) HIP_TRY(hipMalloc(&b->d_gnb, (size_t)b->grid * b->shape.max_n * sizeof(uint16_t)));
+  b->grid = grid_for(b->cus, b->shape.cut.lds, b->shape.cut.nt, b->n_items);
+  if (!b->shape.lo.empty() && !b->shape.lo[0].pairs_in_lds) HIP_TRY(hipMalloc(&b->d_ws, (size_t)b->grid * b->shape.max_n2 * sizeof(uint16_t)));
   return DTO_OK;
 }
 
@@ -259,7 +222,7 @@ int dto_batch_create(dto_job *const *jobs, const uint64_t *n_perm, uint64_t n_jo
       delete b;
       return fail(DTO_ERR_INVALID_ARGUMENT, "bad job or permutation count");
     }
-    if ((rc = ensure_resident(jobs[i]))) {
+    if ((rc = ensure_resident(jobs[i])) || (rc = ensure_cut(jobs[i], 0))) {
       delete b;
       return rc;
     }
@@ -273,7 +236,6 @@ int dto_batch_create(dto_job *const *jobs, const uint64_t *n_perm, uint64_t n_jo
     dto_batch_destroy(b);
     return fail(DTO_ERR_DEVICE, "hipMalloc failed for batch buffers");
   }
-  b->shape.nt = 512;
   if ((rc = batch_plan(b))) {
     dto_batch_destroy(b);
     return rc;
@@ -293,8 +255,7 @@ int dto_batch_launch(dto_batch *b, void *stream) {
   if (!b->exec) {
     /* capture queue reset + persistent kernel once, replay afterwards */
     HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    hipError_t e = launch_batch(b->shape, b->grid, st, b->d_jobs, b->d_items, b->n_items, b->seed, b->d_counter,
-                                b->d_err, batch_globals(b));
+    hipError_t e = batch_kernels(b, st);
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(st, &g);
     if (e != hipSuccess || e2 != hipSuccess) {
@@ -325,47 +286,38 @@ int dto_batch_results(dto_batch *b, dto_result *results) {
   return DTO_OK;
 }
 
-/* Times each candidate launch shape (threads per workgroup x tasks per work
- * item) on this batch and keeps the fastest. */
+/* Times each candidate number of tasks per work item on this batch and keeps
+ * the fastest (the workgroup size follows from the jobs' sizes). */
 int dto_batch_autotune(dto_batch *b, int *waves) {
   if (!b) return fail(DTO_ERR_INVALID_ARGUMENT, "null batch");
-  const int nts[2] = {256, 512};
   const uint32_t chunks[3] = {1, 4, 16};
   float best = 1e30f;
-  int best_nt = b->shape.nt;
   uint32_t best_chunk = b->chunk;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
-  for (int nt : nts) {
-    for (uint32_t c : chunks) {
-      b->shape.nt = nt;
-      b->chunk = c;
-      if (batch_plan(b)) continue;
-      float ms = 0.f;
-      bool good = true;
-      for (int rep = 0; rep < 2 && good; ++rep) {
-        HIP_TRY(hipEventRecord(e0, 0));
-        if (launch_batch(b->shape, b->grid, 0, b->d_jobs, b->d_items, b->n_items, b->seed, b->d_counter, b->d_err,
-                         batch_globals(b)) != hipSuccess)
-          good = false;
-        HIP_TRY(hipEventRecord(e1, 0));
-        HIP_TRY(hipEventSynchronize(e1));
-        HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-      }
-      if (good && ms < best) {
-        best = ms;
-        best_nt = nt;
-        best_chunk = c;
-      }
+  for (uint32_t c : chunks) {
+    b->chunk = c;
+    if (batch_plan(b)) continue;
+    float ms = 0.f;
+    bool good = true;
+    for (int rep = 0; rep < 2 && good; ++rep) {
+      HIP_TRY(hipEventRecord(e0, 0));
+      if (batch_kernels(b, 0) != hipSuccess) good = false;
+      HIP_TRY(hipEventRecord(e1, 0));
+      HIP_TRY(hipEventSynchronize(e1));
+      HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+    }
+    if (good && ms < best) {
+      best = ms;
+      best_chunk = c;
     }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  b->shape.nt = best_nt;
   b->chunk = best_chunk;
   int rc = batch_plan(b);
-  if (waves) *waves = best_nt / 64;
+  if (waves) *waves = b->shape.cut.nt / 64;
   return rc;
 }
 
@@ -524,7 +476,7 @@ static void server_free_request(dto_server *sv, Request *r) {
   if (r->out_off != kNoRegion) sv->pool.release(r->out_off, r->out_bytes);
   if (r->job_off != kNoRegion) sv->pool.release(r->job_off, r->job_bytes);
   if (r->job) {
-    if (r->job->arena || r->job->ws || r->job->gnb)
+    if (r->job->arena || r->job->ws || r->job->cut)
       sv->graveyard.push_back(r->job); /* its hipFree would wait for the device */
     else
       dto_job_destroy(r->job);
@@ -647,21 +599,16 @@ static int server_launch_slice(dto_server *sv, Slot &s) {
   if (sv->up_any) HIP_TRY(hipStreamWaitEvent(s.st, sv->up_ev, 0));
   HIP_TRY(hipMemcpyAsync(s.d_jobs, s.h_jobs, s.parts.size() * sizeof(BatchJob), hipMemcpyHostToDevice, s.st));
   HIP_TRY(hipMemcpyAsync(s.d_items, s.h_items, n_items * sizeof(WorkItem), hipMemcpyHostToDevice, s.st));
-  Shape shape;
-  shape.nt = kNT;
-  shape.hl = cls.hl;
-  shape.pl = cls.pl;
-  shape.nbl = cls.nbl;
-  shape.rc = cls.rc;
-  shape.lds = lds;
-  shape.max_n2 = max_n2;
-  shape.max_n = max_n;
   Globals g;
   g.ws = cls.pl ? nullptr : (uint16_t *)(sv->pool.base + s.ws_off);
   g.ws_stride = max_n2;
   g.gnb = cls.nbl ? nullptr : (uint16_t *)(sv->pool.base + s.gnb_off);
   g.gnb_stride = max_n;
-  hipError_t e = launch_batch(shape, grid, s.st, s.d_jobs, s.d_items, n_items, sv->cfg.seed, s.d_counter, s.d_err, g);
+  hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, s.st, s.d_counter, s.d_err);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = launch_slice(cls.hl, cls.nbl, cls.pl, cls.rc, grid, lds, s.st, s.d_jobs, s.d_items, n_items, sv->cfg.seed,
+                     s.d_counter, s.d_err, g);
   if (e != hipSuccess) return fail(DTO_ERR_DEVICE, std::string("slice launch: ") + hipGetErrorString(e));
   HIP_TRY(hipMemcpyAsync(s.h_err, s.d_err, sizeof(int), hipMemcpyDeviceToHost, s.st));
   HIP_TRY(hipEventRecord(s.ev, s.st));

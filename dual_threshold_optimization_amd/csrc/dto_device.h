@@ -14,6 +14,10 @@ namespace dto {
 
 constexpr uint32_t kBinNone = 0xFFFFu; /* (a,b) pair outside the grid */
 
+/* Levels of the cut tables, and the one a permutation's sweep starts with. */
+constexpr uint32_t kCutLevels = 12;
+constexpr uint32_t kCutStart = 5;
+
 struct DevJob {
   uint32_t N;        /* population size */
   uint32_t N1, N2;   /* list lengths */
@@ -36,6 +40,9 @@ struct DevJob {
   const float *H32;         /* [N+1] LF[x] - x*(ln N - 1), rounded to f32 */
   const float *A32;         /* [T1] H(K_i) + H(N-K_i) */
   const float *B32;         /* [T2] H(n_j) + H(N-n_j) - H(N) */
+  const uint32_t *cut;      /* the cut tables of the screened kernels (dto_cut.h) */
+  uint32_t cut_segs;        /* column segments per row in them */
+  float cut_level[kCutLevels]; /* log p level of each, falling; 0: p == 1 cells only */
   unsigned long long *stats; /* [16] work counters (dto_internal_stats) */
 };
 
@@ -45,6 +52,7 @@ struct LdsLayout {
   uint32_t pairs;    /* u16[N2] row of each list2 position's pair (staging): aliases h; always 0 */
   uint32_t pairs_in_lds;
   uint32_t nb;       /* u16[max(N1,N2)]: list1 bins after the shuffle, then row-sorted list2 bins (nb_in_lds) */
+  uint32_t join;     /* u16[N2] the join (cut kernels with pairs in registers) */
   uint32_t rowstart; /* u32[T1+1] */
   uint32_t cursor;   /* u32[T1] */
   uint32_t cw;       /* u32[W][T2w_pad] per-wave running column counts (2 x u16 per word) */

@@ -34,6 +34,16 @@ LdsLayout make_layout(const HostJob &h, int W, bool with_h, size_t lds_limit, bo
 /* The screened kernels' layout for a job: table and bins in LDS when they
  * fit, else the table in LDS and the bins global, else the table global. */
 LdsLayout screen_layout(const HostJob &h, int W, size_t lds_limit);
+/* The cut kernels (dto_cut.h): how pairs are built, the layout at W waves
+ * (false: the job's lists rule the build out), the shape taken for a set of
+ * jobs, and the levels of a job's cut tables. */
+bool cut_layout(const HostJob &h, int W, int build, LdsLayout *out);
+struct CutShape {
+  int nt = 0, build = 0;
+  uint32_t lds = 0; /* the largest layout's */
+};
+int cut_shape(const HostJob *const *jobs, size_t n, size_t lds_limit, CutShape *out);
+void cut_levels(const HostJob &h, DevJob &d);
 }  // namespace dto
 
 constexpr uint32_t kCounterRing = 256;
@@ -62,9 +72,12 @@ struct dto_job {
   uint32_t *d_ctr = nullptr;
   std::atomic<uint32_t> ctr_next{0};
   int device = -1;
-  dto::LdsLayout lo_screen{}, lo_plain{};
+  dto::LdsLayout lo_screen{}, lo_plain{}; /* lo_screen: a server's slices */
+  dto::CutShape cut_sh{};
+  dto::LdsLayout lo_cut{};
+  void *cut = nullptr; /* the cut tables (dev.cut), set under cut_mu */
+  std::mutex cut_mu;
   uint16_t *ws = nullptr; /* global pair staging (only when the LDS cannot hold the pairs) */
-  uint16_t *gnb = nullptr; /* global bins arrays, one per workgroup (only when lo_screen.nb_in_lds == 0) */
   uint32_t ws_slots = 0;
   /* launches using ws run in order: each waits for the previous one's event */
   hipEvent_t ws_ev = nullptr;
@@ -80,10 +93,46 @@ void bind_job(dto_job *j, unsigned char *base);
 /* Uploads a deferred job into its own arena on first use; fails when the
  * job sits in a server's pool (the server owns it). */
 int ensure_resident(dto_job *j);
+/* Launches that stage their pairs in the job's global buffer (lists too long
+ * for the LDS) run one after another, whatever their streams: each waits for
+ * the previous one's completion event.  Inside a stream capture the wait is
+ * left out (a capture cannot wait on work recorded outside it), so captured
+ * launches of one such job must not overlap. */
+struct StagingOrder {
+  dto_job *j;
+  hipStream_t st;
+  bool on = false;
+  StagingOrder(const dto_job *job, const dto::LdsLayout &lo, hipStream_t s) : j(const_cast<dto_job *>(job)), st(s) {
+    if (lo.pairs_in_lds || !j->ws_ev) return;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+    if (cs != hipStreamCaptureStatusNone) return;
+    j->ws_mu.lock();
+    on = true;
+    if (j->ws_used) (void)hipStreamWaitEvent(st, j->ws_ev, 0);
+  }
+  ~StagingOrder() {
+    if (!on) return;
+    if (hipEventRecord(j->ws_ev, st) == hipSuccess) j->ws_used = true;
+    j->ws_mu.unlock();
+  }
+};
+
 namespace dto {
 /* The debug grid of one permutation on a stream (k_grid_counts then
  * k_grid_pvalues): overlap counts into kcnt (T1 * T2 words), every cell's
  * record into out; an out-of-range permutation index sets *err. */
 hipError_t launch_grid(dto_job *job, const uint32_t *d1, const uint32_t *d2, uint32_t *kcnt, dto_record *out, int *err,
                        hipStream_t st);
+/* Builds a job's cut tables on a stream if it has none yet; they are complete
+ * on return. */
+int ensure_cut(dto_job *j, hipStream_t st);
+hipError_t launch_cut(dto_job *j, bool expl, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
+                      uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted, uint32_t lead,
+                      dto_record *out);
+struct BatchJob;
+struct WorkItem;
+hipError_t launch_batch_cut(const CutShape &sh, uint32_t grid, hipStream_t st, const BatchJob *jobs,
+                            const WorkItem *items, uint32_t n_items, uint64_t seed, uint32_t *counter, int *err,
+                            uint16_t *ws, uint32_t ws_stride);
 }  // namespace dto

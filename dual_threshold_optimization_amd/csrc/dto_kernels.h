@@ -304,40 +304,52 @@ __device__ __forceinline__ void load_job_tables(const DevJob &J, const Lds &S) {
 }
 
 /* Visits the Philox permutation of one list, idx[k] for every k < n, spread
- * over the workgroup.  The domain goes in chunks of NT * kShufU consecutive
- * elements, each thread evaluating kShufU consecutive ones; a workgroup
- * prefix count (wave scan + per-wave totals in wsum[W]) ranks those that
- * fall below n.  Every thread runs every chunk and hands fn its kShufU
- * (rank, value) pairs at once, fn(rank[], value[]), value >= n marking an
- * element outside [0, n), so that fn can issue all its loads together. */
+ * over the workgroup.  The domain goes in chunks of NT * kShufU elements; of a
+ * chunk, each wave takes 64 * kShufU consecutive ones, kShufU per lane, 64
+ * apart, so that the lanes of one step hold consecutive ranks and their
+ * loads by rank coalesce.  Ballots within the wave and a prefix over the
+ * per-wave totals in wsum[W] rank the elements below n.  Every thread runs
+ * every chunk and hands fn its kShufU (rank, value) pairs at once, fn(rank[],
+ * value[]), value >= n marking an element outside [0, n), so that fn can
+ * issue all its loads together. */
 constexpr uint32_t kShufU = 16;
+template <int NT>
+__device__ __forceinline__ void shuffle_chunk(const Shuffle &s, uint32_t *wsum, uint32_t base, uint32_t &carried,
+                                              uint32_t *rk, uint32_t *v) {
+  constexpr uint32_t W = NT / 64;
+  const uint32_t lane = lane_id(), w = wave_id();
+  const uint32_t p0 = base + w * (64u * kShufU) + lane;
+  uint32_t cnt = 0u; /* elements below n in the wave's earlier steps */
+#pragma unroll
+  for (uint32_t u = 0; u < kShufU; ++u) {
+    const uint32_t p = p0 + 64u * u;
+    if (s.ident)
+      v[u] = min(p, s.n);
+    else
+      v[u] = p < s.dom ? feistel_once(s, p) : s.n;
+    const uint64_t m = __ballot(v[u] < s.n);
+    rk[u] = cnt + mask_lt(m);
+    cnt += (uint32_t)__popcll(m);
+  }
+  if (lane == 0) wsum[w] = cnt;
+  __syncthreads();
+  uint32_t r = carried, total = 0;
+  for (uint32_t x = 0; x < W; ++x) {
+    const uint32_t t = wsum[x];
+    r += x < w ? t : 0u;
+    total += t;
+  }
+  __syncthreads();
+  carried += total;
+#pragma unroll
+  for (uint32_t u = 0; u < kShufU; ++u) rk[u] += r;
+}
 template <int NT, typename Fn>
 __device__ __forceinline__ void shuffle_visit(const Shuffle &s, uint32_t *wsum, Fn fn) {
-  constexpr uint32_t W = NT / 64;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
   uint32_t carried = 0;
   for (uint32_t base = 0; base < s.dom; base += NT * kShufU) {
-    uint32_t v[kShufU], rk[kShufU], cnt = 0;
-#pragma unroll
-    for (uint32_t u = 0; u < kShufU; ++u) {
-      const uint32_t p = base + tid * kShufU + u;
-      v[u] = p < s.dom ? feistel_once(s, p) : s.n;
-      rk[u] = cnt; /* rank among this thread's elements below n */
-      cnt += v[u] < s.n ? 1u : 0u;
-    }
-    const uint32_t ex = wave_excl_scan(cnt);
-    if (lane == 63) wsum[w] = ex + cnt;
-    __syncthreads();
-    uint32_t r = carried + ex, total = 0;
-    for (uint32_t x = 0; x < W; ++x) {
-      const uint32_t t = wsum[x];
-      r += x < w ? t : 0u;
-      total += t;
-    }
-    __syncthreads();
-    carried += total;
-#pragma unroll
-    for (uint32_t u = 0; u < kShufU; ++u) rk[u] += r;
+    uint32_t v[kShufU], rk[kShufU];
+    shuffle_chunk<NT>(s, wsum, base, carried, rk, v);
     fn(rk, v);
   }
 }

@@ -244,12 +244,14 @@ DTO_HD U32x4 philox4x32_10(U32x4 c, uint32_t k0, uint32_t k1) {
 #define DTO_FEISTEL_ROUNDS 8
 struct Shuffle {
   uint32_t n, pa, amask, b, dom;
+  uint32_t ident; /* 1: the identity in the shuffle's place (the unpermuted task) */
   uint32_t rk[DTO_FEISTEL_ROUNDS];
 };
 
 DTO_HD Shuffle shuffle_make(uint64_t seed, uint32_t job, uint32_t perm, uint32_t list, uint32_t n) {
   Shuffle s;
   s.n = n;
+  s.ident = 0;
   uint32_t bl = 0; /* ceil(log2 n) */
   while (bl < 31 && (1u << bl) < n) ++bl;
   if (bl <= 12) {
