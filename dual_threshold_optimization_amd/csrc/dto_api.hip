@@ -246,22 +246,6 @@ int ensure_resident(dto_job *j) {
 /* ------------------------------------------------------------------ */
 /* launches                                                              */
 /* ------------------------------------------------------------------ */
-/* The plain kernel (every cell exact). */
-template <bool E, bool PA>
-static hipError_t launch_opt(const dto_job *j, const LdsLayout &lo, uint32_t grid, hipStream_t st,
-                             const uint32_t *i1, const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed,
-                             uint32_t job_id, int32_t permuted, dto_record *out) {
-  auto kern = k_optimize<kNT, E, false, true, PA, false, true>;
-  (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lo.total);
-  /* a slot of the job's counter ring for this launch, zeroed on its stream */
-  uint32_t *ctr = j->d_ctr + (const_cast<dto_job *>(j)->ctr_next.fetch_add(1u) % kCounterRing);
-  StagingOrder order(j, lo, st);
-  hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, ctr);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(kNT), lo.total, st, j->dev, lo, i1, i2, n_perm, base, seed, job_id,
-                     permuted, out, j->d_err, j->ws, nullptr, ctr);
-  return hipGetLastError();
-}
-
 /* Number of workgroups for a permutation launch: enough to fill every CU at
  * the occupancy the LDS footprint allows, never more than the work. */
 static uint32_t perm_grid(const dto_job *j, const LdsLayout &lo, uint64_t n_perm, uint64_t max_per_cu) {
@@ -283,14 +267,9 @@ static int launch_perms(dto_job *j, uint32_t mode, bool expl, const uint32_t *d1
   if (n_perm >= (1ull << 32) - 65536ull) return fail(DTO_ERR_TOO_LARGE, "too many permutations in one launch");
   hipError_t e;
   if (mode == DTO_MODE_PLAIN) {
-    const LdsLayout &lo = j->lo_plain;
-    const uint32_t g = perm_grid(j, lo, n_perm, 4);
-    if (expl)
-      e = lo.pairs_in_lds ? launch_opt<true, true>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
-                          : launch_opt<true, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
-    else
-      e = lo.pairs_in_lds ? launch_opt<false, true>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out)
-                          : launch_opt<false, false>(j, lo, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
+    /* at most one workgroup per staging slot */
+    const uint32_t g = perm_grid(j, j->lo_plain, ~0ull, 4);
+    e = launch_plain(j, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
   } else if (mode == DTO_MODE_SCREENED) {
     int rc = ensure_cut(j, st);
     if (rc) return rc;
@@ -338,33 +317,6 @@ struct DevBuf {
     if (p) (void)hipFree(p);
   }
 };
-
-/* The debug grid of one permutation on a stream: overlap counts into kcnt
- * (T1 * T2 words), then every cell's exact record into out; an out-of-range
- * permutation index sets *err. */
-hipError_t dto::launch_grid(dto_job *job, const uint32_t *d1, const uint32_t *d2, uint32_t *kcnt, dto_record *out,
-                              int *err, hipStream_t st) {
-  const size_t cells = (size_t)job->dev.T1 * job->dev.T2;
-  const LdsLayout &lo = job->lo_plain;
-  if (lo.pairs_in_lds) {
-    (void)hipFuncSetAttribute((const void *)k_grid_counts<kNT, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)lo.total);
-    hipLaunchKernelGGL((k_grid_counts<kNT, true>), dim3(1), dim3(kNT), lo.total, st, job->dev, lo, d1, d2, kcnt, err,
-                       job->ws);
-  } else {
-    (void)hipFuncSetAttribute((const void *)k_grid_counts<kNT, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)lo.total);
-    StagingOrder order(job, lo, st);
-    hipLaunchKernelGGL((k_grid_counts<kNT, false>), dim3(1), dim3(kNT), lo.total, st, job->dev, lo, d1, d2, kcnt,
-                       err, job->ws);
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int32_t permuted = (d1 || d2) ? 1 : 0;
-  const uint32_t g = (uint32_t)std::min<size_t>((cells + 255) / 256, 8192);
-  hipLaunchKernelGGL(k_grid_pvalues, dim3(g), dim3(256), 0, st, job->dev, (const uint32_t *)kcnt, permuted, out);
-  return hipGetLastError();
-}
 
 /* ------------------------------------------------------------------ */
 /* C ABI                                                                  */
@@ -613,6 +565,7 @@ void dto_job_destroy(dto_job *job) {
   if (job->arena) (void)hipFree(job->arena);
   if (job->ws) (void)hipFree(job->ws);
   if (job->cut) (void)hipFree(job->cut);
+  if (job->partial) (void)hipFree(job->partial);
   if (job->ws_ev) (void)hipEventDestroy(job->ws_ev);
   delete job;
 }

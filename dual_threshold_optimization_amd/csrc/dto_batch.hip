@@ -476,7 +476,7 @@ static void server_free_request(dto_server *sv, Request *r) {
   if (r->out_off != kNoRegion) sv->pool.release(r->out_off, r->out_bytes);
   if (r->job_off != kNoRegion) sv->pool.release(r->job_off, r->job_bytes);
   if (r->job) {
-    if (r->job->arena || r->job->ws || r->job->cut)
+    if (r->job->arena || r->job->ws || r->job->cut || r->job->partial)
       sv->graveyard.push_back(r->job); /* its hipFree would wait for the device */
     else
       dto_job_destroy(r->job);

@@ -76,6 +76,7 @@ struct dto_job {
   dto::CutShape cut_sh{};
   dto::LdsLayout lo_cut{};
   void *cut = nullptr; /* the cut tables (dev.cut), set under cut_mu */
+  void *partial = nullptr; /* split plain launches' partial results, set under cut_mu */
   std::mutex cut_mu;
   uint16_t *ws = nullptr; /* global pair staging (only when the LDS cannot hold the pairs) */
   uint32_t ws_slots = 0;
@@ -130,6 +131,9 @@ int ensure_cut(dto_job *j, hipStream_t st);
 hipError_t launch_cut(dto_job *j, bool expl, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
                       uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted, uint32_t lead,
                       dto_record *out);
+hipError_t launch_plain(dto_job *j, bool expl, uint32_t max_grid, hipStream_t st, const uint32_t *i1,
+                        const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id,
+                        int32_t permuted, dto_record *out);
 struct BatchJob;
 struct WorkItem;
 hipError_t launch_batch_cut(const CutShape &sh, uint32_t grid, hipStream_t st, const BatchJob *jobs,

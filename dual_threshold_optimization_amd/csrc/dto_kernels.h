@@ -578,20 +578,6 @@ __device__ __forceinline__ void add_bins(const Lds &S, uint32_t *C, uint32_t e0,
   }
 }
 
-/* Adds (sign +1) or removes (-1) row i's pairs into a wave's column counts. */
-__device__ __forceinline__ void row_update(const Lds &S, uint32_t *C, uint32_t i, bool add) {
-  const uint32_t lane = lane_id();
-  for (uint32_t e = S.rowstart[i] + lane; e < S.rowstart[i + 1]; e += 64) {
-    uint32_t b = S.nb[e];
-    uint32_t inc = 1u << ((b & 1u) * 16u);
-    if (add)
-      atomicAdd(&C[b >> 1], inc);
-    else
-      atomicSub(&C[b >> 1], inc);
-  }
-  wave_sync();
-}
-
 /* Start of this lane's run of columns: exclusive wave scan of lane totals. */
 __device__ __forceinline__ uint32_t row_lane_offset(const uint32_t *C, uint32_t wbeg, uint32_t c2,
                                                     uint32_t T2w) {
@@ -1227,15 +1213,6 @@ __device__ __forceinline__ ZeroKey class1_best(const DevJob &J, const LdsLayout 
   return wave_zero(o);
 }
 
-/* The launch's task counter and where a workgroup puts its next task; with
- * explicit permutations, their index arrays (for the prefetch). */
-struct NextTask {
-  uint32_t *counter;
-  uint32_t *slot;
-  const uint32_t *idx1, *idx2;
-  uint64_t n_perm;
-};
-
 /* One permutation: overlap grid -> best cell.  Returns the best key in
  * thread 0 (others: undefined).  Rows are interleaved over the waves: every
  * wave adds every row's pairs to its own running column counts, and scans
@@ -1243,30 +1220,16 @@ struct NextTask {
  * empty tail): 1 in, 0 left out (the job cannot have such cells,
  * DevJob.kle), 2 chosen by J.kle at run time (the batch kernel, whose jobs
  * differ). */
-template <int NT, bool EXPLICIT, bool HLDS, bool PLAIN, bool PL, bool REGCOLS, bool NBL = true, int ZCM = 2>
+template <int NT, bool EXPLICIT, bool HLDS, bool PL, bool REGCOLS, bool NBL = true, int ZCM = 2>
 __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayout &Lo, const Lds &S, const uint32_t *i1,
                                  const uint32_t *i2, const Shuffle &s1, const Shuffle &s2, int *err,
-                                 WaveStats &st, uint16_t *gpairs, const NextTask *nt = nullptr) {
+                                 WaveStats &st, uint16_t *gpairs) {
   constexpr uint32_t W = NT / 64;
   const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
   uint64_t tc0 = cycles();
   build_rows<NT, EXPLICIT, HLDS, PL, NBL>(J, Lo, S, i1, i2, s1, s2, err, gpairs);
   uint64_t tc1 = cycles();
   st.cyc[0] += tc1 - tc0;
-  /* wave 0 claims the workgroup's next task once the build is done: by then
-   * every workgroup of the launch has started, so none takes a second task
-   * while another still has none.  The claim does not depend on the grid's
-   * contents, and the slot is read after this task's last barrier, so every
-   * task moves the workgroup on to a new one. */
-  uint32_t pnext = kNone;
-  if (nt && w == 0u) {
-    if (lane == 0) {
-      pnext = atomicAdd(nt->counter, 1u);
-      *nt->slot = pnext;
-    }
-    pnext = (uint32_t)__builtin_amdgcn_readfirstlane((int)pnext);
-  }
-
   const uint32_t T1 = J.T1, T2 = J.T2, T2w = J.T2w;
   uint32_t *C = S.cw + w * Lo.T2w_pad;
   /* count words per lane; wide grids (several segments per row) take an odd
@@ -1276,39 +1239,6 @@ __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayou
   const uint32_t c2 = REGCOLS ? (T2w + 63) / 64 : ((T2w + 63) / 64) | 1u;
   const uint32_t wbeg = lane * c2;
   const char *Hb = HLDS ? (const char *)S.h : (const char *)J.H32;
-
-  if (PLAIN) {
-    BestKey xb = no_best();
-    uint32_t added = 0;
-    for (uint32_t i = w; i < T1; i += W) {
-      rows_update<NBL>(S, C, added, i + 1, true);
-      added = i + 1;
-      const uint32_t K = J.K[i];
-      uint32_t run = row_lane_offset(C, wbeg, c2, T2w);
-#pragma unroll 1
-      for (uint32_t t = 0; t < c2; ++t) {
-        const uint32_t wi = wbeg + t;
-        const uint32_t x = wi < T2w ? C[wi] : 0u;
-#pragma unroll 1
-        for (uint32_t h = 0; h < 2; ++h) {
-          const uint32_t j = 2 * wi + h;
-          run += h ? (x >> 16) : (x & 0xFFFFu);
-          if (j >= T2) continue;
-          const uint32_t k = run;
-          double p = dto_tail_exact(J.LF, J.N, K, S.coln[j], k, J.D[j], S.tab, nullptr);
-          take_better(xb, p, k, (i << 16) | j);
-        }
-      }
-    }
-    xb = wave_best(xb);
-    if (lane == 0) S.redB[2 * W + w] = xb;
-    __syncthreads();
-    BestKey b = no_best();
-    if (tid == 0)
-      for (uint32_t v = 0; v < W; ++v) merge_best(b, S.redB[2 * W + v]);
-    __syncthreads();
-    return b;
-  }
 
   /* this lane's column constants, kept in registers across rows; columns
    * past T2 repeat the last column's n (their k equals its k) and get no cell */
@@ -1359,7 +1289,6 @@ __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayou
    * one load per 64 rows instead of a global load latency per row */
   uint32_t Kl = 0u, NKl = 0u; /* K_i and 4 (N - K_i) */
   float Al = 0.f;
-  uint32_t pfacc = 0u; /* keeps the prefetch loads */
   for (uint32_t i = w, q = 0; i < T1; i += W, ++q) {
     if ((q & 63u) == 0u) {
       const uint32_t ir = i + lane * W;
@@ -1590,25 +1519,6 @@ __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayou
   if (nc) flush_candidates<NT>(J, S, cand, nc, c3, n3, xb, Uw, U2w, st);
   uint64_t tc4 = cycles();
   st.cyc[3] += tc4 - tc3;
-  if (nt && w == 0u && nt->idx1 && nt->idx2 && pnext < nt->n_perm) {
-    /* the next task's index arrays, late in this task so that they are
-     * still in the cache when its build reads them: one load per 128-byte
-     * line, kPf lines per lane issued together before a single wait (the
-     * sum keeps the loads) */
-    constexpr uint32_t kPf = 16;
-    const uint32_t *p1 = nt->idx1 + (uint64_t)pnext * J.N1, *p2 = nt->idx2 + (uint64_t)pnext * J.N2;
-    const uint32_t l1 = (J.N1 + 31u) / 32u, l2 = (J.N2 + 31u) / 32u;
-    for (uint32_t t0 = 0; t0 < l1 + l2; t0 += 64u * kPf) {
-      uint32_t v[kPf];
-#pragma unroll
-      for (uint32_t u = 0; u < kPf; ++u) {
-        const uint32_t t = t0 + u * 64u + lane;
-        v[u] = t < l1 ? p1[32u * t] : (t < l1 + l2 ? p2[32u * (t - l1)] : 0u);
-      }
-#pragma unroll
-      for (uint32_t u = 0; u < kPf; ++u) pfacc += v[u];
-    }
-  }
   /* tier 3: exact FP64 for cells whose bracket reaches the best bound this
    * wave knows of (its own, and what the other waves have shared so far: no
    * barrier, a looser bound only evaluates more cells) */
@@ -1622,7 +1532,6 @@ __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayou
   st.cyc[4] += cycles() - tc5;
   if (lane == 0) S.redB[2 * W + w] = xb;
   __syncthreads();
-  if (pfacc == 0xFFFFFFFFu && J.N == 0u) S.redS[0] = pfacc; /* never true: N >= 1 */
   /* p == 1 cells matter only when no cell has p < 1 */
   bool need1 = true;
   for (uint32_t v = 0; v < W; ++v) {
@@ -1699,59 +1608,6 @@ __device__ __forceinline__ void write_record(const DevJob &J, const BestKey &b, 
   r.idx2 = j;
   r.ties = (b.np < 0xFFFFu ? b.np : 0xFFFFu) | ((b.npk < 0xFFFFu ? b.npk : 0xFFFFu) << 16);
   *out = r;
-}
-
-/* Permutations [perm_base, perm_base + n_perm) of one job.  EXPLICIT: idx1 /
- * idx2 hold n_perm permutations back to back (NULL: identity); otherwise the
- * Philox shuffle keyed by (seed, job_id, permutation id, list).  ws: per
- * workgroup pair staging (N2 u16 each) when !PL.  Workgroups take
- * permutations from a device counter (zeroed before the launch), so that
- * permutations of uneven cost spread evenly; every workgroup exits once the
- * counter passes n_perm.  The screen keeps its k > K test for every job:
- * one code path in the sweeps costs less than leaving the test out. */
-template <int NT, bool EXPLICIT, bool HLDS, bool PLAIN, bool PL, bool REGCOLS, bool NBL>
-__global__ __launch_bounds__(NT) void k_optimize(DevJob J, LdsLayout Lo, const uint32_t *__restrict__ idx1,
-                                                 const uint32_t *__restrict__ idx2, uint64_t n_perm,
-                                                 uint64_t perm_base, uint64_t seed, uint32_t job_id,
-                                                 int32_t permuted, dto_record *__restrict__ out,
-                                                 int *__restrict__ err, uint16_t *__restrict__ ws,
-                                                 uint16_t *__restrict__ gnb, uint32_t *__restrict__ counter) {
-  /* no static LDS here: the dynamic region then starts at address 0 */
-  extern __shared__ __align__(16) unsigned char smem[];
-  uint32_t &s_next = *(uint32_t *)(smem + Lo.misc);
-  constexpr int W = NT / 64;
-  const Lds S = lds_view<NBL>(smem, Lo, W, NBL ? nullptr : gnb + (uint64_t)blockIdx.x * max(J.N1, J.N2));
-  load_job_tables<NT, HLDS>(J, S);
-  __syncthreads();
-  uint16_t *gpairs = PL ? nullptr : ws + (uint64_t)blockIdx.x * J.N2;
-  WaveStats st = {0u, 0u, 0u, {0, 0, 0, 0, 0}, 0u, 0u, 0u, 0u, 0u};
-  /* the first task; each task claims the next one (optimize_perm) */
-  if (threadIdx.x == 0) s_next = atomicAdd(counter, 1u);
-  __syncthreads();
-  uint64_t pp = s_next;
-  __syncthreads();
-  const NextTask nt = {counter, &s_next, EXPLICIT && !PLAIN ? idx1 : nullptr, EXPLICIT && !PLAIN ? idx2 : nullptr,
-                       n_perm};
-  for (;;) {
-    if (pp >= n_perm) break;
-    const uint64_t pid = perm_base + pp;
-    const uint32_t *i1 = (EXPLICIT && idx1) ? idx1 + pp * J.N1 : nullptr;
-    const uint32_t *i2 = (EXPLICIT && idx2) ? idx2 + pp * J.N2 : nullptr;
-    Shuffle s1, s2;
-    if (!EXPLICIT) {
-      s1 = shuffle_make(seed, job_id, (uint32_t)pid, 1u, J.N1);
-      s2 = shuffle_make(seed, job_id, (uint32_t)pid, 2u, J.N2);
-    }
-    BestKey b =
-        optimize_perm<NT, EXPLICIT, HLDS, PLAIN, PL, REGCOLS, NBL, 1>(J, Lo, S, i1, i2, s1, s2, err, st, gpairs, &nt);
-    /* a counter value claimed during this task (optimize_perm claims one
-     * every time, after the build): published by its last barrier, and new,
-     * so the loop always moves on */
-    const uint64_t pn = s_next;
-    if (threadIdx.x == 0) write_record(J, b, permuted, out + pp, err);
-    pp = pn;
-  }
-  flush_stats(J, st);
 }
 
 /* Zeroes one work counter (a kernel, not a memset, so that callers may
@@ -1831,63 +1687,14 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchJob *__restrict__ jobs,
       BestKey b;
       Shuffle s1, s2;
       if (t == 0) {
-        b = optimize_perm<NT, true, HLDS, false, PL, REGCOLS, NBL>(B.J, B.lo, S, nullptr, nullptr, s1, s2, err, st,
-                                                                  gpairs);
+        b = optimize_perm<NT, true, HLDS, PL, REGCOLS, NBL>(B.J, B.lo, S, nullptr, nullptr, s1, s2, err, st, gpairs);
       } else {
         s1 = shuffle_make(seed, B.job_id, t - 1, 1u, B.J.N1);
         s2 = shuffle_make(seed, B.job_id, t - 1, 2u, B.J.N2);
-        b = optimize_perm<NT, false, HLDS, false, PL, REGCOLS, NBL>(B.J, B.lo, S, nullptr, nullptr, s1, s2, err, st,
-                                                                   gpairs);
+        b = optimize_perm<NT, false, HLDS, PL, REGCOLS, NBL>(B.J, B.lo, S, nullptr, nullptr, s1, s2, err, st, gpairs);
       }
       if (threadIdx.x == 0) write_record(B.J, b, t == 0 ? 0 : 1, B.out + t, err);
     }
-  }
-}
-
-/* Overlap counts of every cell for one permutation (debug grid export). */
-template <int NT, bool PL>
-__global__ __launch_bounds__(NT) void k_grid_counts(DevJob J, LdsLayout Lo, const uint32_t *__restrict__ idx1,
-                                                    const uint32_t *__restrict__ idx2,
-                                                    uint32_t *__restrict__ kout, int *__restrict__ err,
-                                                    uint16_t *__restrict__ ws) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int W = NT / 64;
-  const Lds S = lds_view(smem, Lo, W);
-  Shuffle s1, s2;
-  build_rows<NT, true, false, PL>(J, Lo, S, idx1, idx2, s1, s2, err, ws);
-  const uint32_t w = wave_id(), lane = lane_id();
-  const uint32_t T1 = J.T1, T2 = J.T2, T2w = J.T2w;
-  uint32_t *C = S.cw + w * Lo.T2w_pad;
-  const uint32_t c2 = (T2w + 63) / 64, wbeg = lane * c2;
-  for (uint32_t i = 0; i < T1; ++i) {
-    row_update(S, C, i, true);
-    if (i % W != w) continue;
-    uint32_t run = row_lane_offset(C, wbeg, c2, T2w);
-    for (uint32_t t = 0; t < c2; ++t) {
-      const uint32_t wi = wbeg + t;
-      const uint32_t x = wi < T2w ? C[wi] : 0u;
-      for (uint32_t h = 0; h < 2; ++h) {
-        const uint32_t j = 2 * wi + h;
-        run += h ? (x >> 16) : (x & 0xFFFFu);
-        if (j < T2) kout[(uint64_t)i * T2 + j] = run;
-      }
-    }
-  }
-}
-
-/* Exact p-value of every cell from the count grid (debug grid export). */
-static __global__ __launch_bounds__(256) void k_grid_pvalues(DevJob J, const uint32_t *__restrict__ kin,
-                                                      int32_t permuted, dto_record *__restrict__ out) {
-  __shared__ uint64_t tab[256];
-  tab[threadIdx.x] = kExpTabC[threadIdx.x];
-  __syncthreads();
-  const uint64_t cells = (uint64_t)J.T1 * J.T2;
-  for (uint64_t c = (uint64_t)blockIdx.x * 256 + threadIdx.x; c < cells; c += (uint64_t)gridDim.x * 256) {
-    const uint32_t i = (uint32_t)(c / J.T2), j = (uint32_t)(c % J.T2);
-    const uint32_t k = kin[c];
-    double p = dto_tail_exact(J.LF, J.N, J.K[i], J.n[j], k, J.D[j], tab, nullptr);
-    BestKey b = {p, k, (i << 16) | j};
-    write_record(J, b, permuted, out + c, nullptr);
   }
 }
 
