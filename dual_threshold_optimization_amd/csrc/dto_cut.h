@@ -141,13 +141,18 @@ __device__ __forceinline__ void load_cut_tables(const DevJob &J, const LdsLayout
  * shuffle domains at most kRegPairs * NT elements, no repeated ids).  What
  * bounds the build is the gather of the join at random positions: from L2
  * it is one cache line a lane; the LDS answers 64 lanes in a few cycles.
- * The pairs' staging in registers is what leaves the LDS room for it. */
+ * The pairs' staging in registers is what leaves the LDS room for it.  Loads
+ * take clamped indices instead of conditions: under a condition each load
+ * is a basic block of its own and its wait comes before the next one. */
 template <int NT, bool EXPLICIT>
 __device__ __forceinline__ void build_regs(const DevJob &J, const LdsLayout &Lo, const Lds &S, const uint16_t *jn,
                                            const uint32_t *i1, const uint32_t *i2, const Shuffle &s1,
                                            const Shuffle &s2, int *err) {
   constexpr uint32_t W = NT / 64, U = kShufU, CH = kRegPairs / U;
-  const uint32_t tid = threadIdx.x;
+  uint32_t tid = threadIdx.x;
+  /* opaque: else the positions and addresses of every element, the same in
+   * every task, are computed before the task loop and kept in scratch */
+  asm volatile("" : "+v"(tid));
   const uint32_t T1 = J.T1, T2 = J.T2, N1 = J.N1, N2 = J.N2, T2wp = Lo.T2w_pad;
   const uint16_t *bin1 = J.bin1, *bin2 = J.bin2;
   for (uint32_t t = tid; t <= T1; t += NT) S.rowstart[t] = 0;
@@ -160,22 +165,25 @@ __device__ __forceinline__ void build_regs(const DevJob &J, const LdsLayout &Lo,
     uint32_t k[U], m[U], bn[U];
     if (EXPLICIT) {
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) {
-        k[u] = base + u * NT + tid;
-        m[u] = N1;
-        if (k[u] < N1) {
-          m[u] = i1 ? i1[k[u]] : k[u];
-          if (m[u] >= N1) atomicOr(err, 1);
-        }
+      for (uint32_t u = 0; u < U; ++u) k[u] = base + u * NT + tid;
+      if (i1) {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) m[u] = at32(i1, min(k[u], N1 - 1u));
+      } else {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) m[u] = k[u];
       }
     } else {
       shuffle_chunk<NT>(s1, S.redS, base, carried, k, m);
     }
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) bn[u] = m[u] < N1 ? bin1[k[u]] : 0u;
+    for (uint32_t u = 0; u < U; ++u) bn[u] = at32(bin1, min(k[u], N1 - 1u));
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u)
-      if (m[u] < N1) S.nb[m[u]] = (uint16_t)bn[u];
+    for (uint32_t u = 0; u < U; ++u) {
+      const bool in = EXPLICIT ? k[u] < N1 : true;
+      if (EXPLICIT && in && m[u] >= N1) atomicOr(err, 1);
+      if (in && m[u] < N1) S.nb[m[u]] = (uint16_t)bn[u];
+    }
   }
   __syncthreads();
   /* pairs (a << 16 | b) per list-2 position, counted per row */
@@ -186,27 +194,39 @@ __device__ __forceinline__ void build_regs(const DevJob &J, const LdsLayout &Lo,
 #pragma unroll
     for (uint32_t u = 0; u < U; ++u) pr[c * U + u] = kNone;
     if (c * NT * U < (EXPLICIT ? N2 : s2.dom)) {
-      uint32_t e[U], q[U], b[U];
+      uint32_t e[U], q[U], b[U], a[U];
       if (EXPLICIT) {
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
-          e[u] = (c * U + u) * NT + tid;
-          q[u] = N2;
-          if (e[u] < N2) {
-            q[u] = i2 ? i2[e[u]] : e[u];
-            if (q[u] >= N2) atomicOr(err, 1);
-          }
+        for (uint32_t u = 0; u < U; ++u) e[u] = (c * U + u) * NT + tid;
+        if (i2) {
+#pragma unroll
+          for (uint32_t u = 0; u < U; ++u) q[u] = at32(i2, min(e[u], N2 - 1u));
+        } else {
+#pragma unroll
+          for (uint32_t u = 0; u < U; ++u) q[u] = e[u];
         }
       } else {
         shuffle_chunk<NT>(s2, S.redS, c * NT * U, carried, e, q);
       }
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) b[u] = q[u] < N2 ? bin2[e[u]] : kBinNone;
-      uint32_t a[U];
+      for (uint32_t u = 0; u < U; ++u) b[u] = at32(bin2, min(e[u], N2 - 1u));
+      if (EXPLICIT) {
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) a[u] = q[u] < N2 ? jn[q[u]] : 0xFFFFu;
+        for (uint32_t u = 0; u < U; ++u) {
+          if (e[u] < N2 && q[u] >= N2) atomicOr(err, 1);
+          q[u] = e[u] < N2 ? q[u] : N2;
+        }
+      }
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) a[u] = a[u] != 0xFFFFu ? S.nb[a[u]] : kBinNone;
+      for (uint32_t u = 0; u < U; ++u) a[u] = jn[min(q[u], N2 - 1u)];
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) a[u] = q[u] < N2 ? a[u] : 0xFFFFu;
+      /* positions without a partner read entry 0, and are left out */
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t x = S.nb[a[u] != 0xFFFFu ? a[u] : 0u];
+        a[u] = a[u] != 0xFFFFu ? x : kBinNone;
+      }
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u)
         if (a[u] < T1 && b[u] < T2) {
@@ -573,6 +593,7 @@ __global__ __launch_bounds__(NT, 4) void k_cut(DevJob J, LdsLayout Lo, const uin
     /* the value claimed during this task, published by its barriers */
     const uint64_t pn = s_next;
     if (threadIdx.x == 0) write_record(J, b, first ? 0 : permuted, out + pp, err);
+    wave_sync(); /* keeps thread 0's block apart from the next iteration's (see k_plain) */
     pp = pn;
   }
   flush_stats(J, st);
@@ -610,6 +631,7 @@ __global__ __launch_bounds__(NT, 4) void k_batch_cut(const BatchJob *__restrict_
       const BestKey b =
           optimize_cut<NT, false, BUILD>(B.J, B.lo, S, nullptr, nullptr, s1, s2, err, st, smem, gpairs, nullptr, nullptr);
       if (threadIdx.x == 0) write_record(B.J, b, t == 0 ? 0 : 1, B.out + t, err);
+      wave_sync(); /* keeps thread 0's block apart from the next iteration's (see k_plain) */
     }
   }
 }

@@ -354,6 +354,12 @@ __device__ __forceinline__ void shuffle_visit(const Shuffle &s, uint32_t *wsum, 
   }
 }
 
+/* p[i] with a 32-bit byte offset, which a load adds to a scalar base. */
+template <typename T>
+__device__ __forceinline__ T at32(const T *p, uint32_t i) {
+  return *(const T *)((const char *)p + i * (uint32_t)sizeof(T));
+}
+
 /* Phases A-B for one permutation: leaves the row-sorted list2 bins in S.nb,
  * row offsets in S.rowstart and zeroed per-wave column counts.  Each list2
  * position's pair is staged in `pairs`: with HLDS in the screen-table region
@@ -366,7 +372,10 @@ __device__ __forceinline__ void build_rows(const DevJob &J, const LdsLayout &Lo,
                                            const uint32_t *i2, const Shuffle &s1, const Shuffle &s2, int *err,
                                            uint16_t *gpairs) {
   constexpr int W = NT / 64;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
+  uint32_t tid = threadIdx.x;
+  /* opaque: else the positions and addresses of every element, the same in
+   * every task, are computed before the task loop and kept in scratch */
+  asm volatile("" : "+v"(tid));
   const uint32_t T1 = J.T1, T2 = J.T2, T2wp = Lo.T2w_pad;
   uint16_t *lpairs = S.pairs;
   uint16_t *vpairs = gpairs; /* global staging, read back by other waves after a barrier */
@@ -386,7 +395,7 @@ __device__ __forceinline__ void build_rows(const DevJob &J, const LdsLayout &Lo,
     shuffle_visit<NT>(s1, S.redS, [&](const uint32_t *k, const uint32_t *m) {
       uint32_t bn[kShufU];
 #pragma unroll
-      for (uint32_t u = 0; u < kShufU; ++u) bn[u] = m[u] < J.N1 ? bin1[k[u]] : 0u;
+      for (uint32_t u = 0; u < kShufU; ++u) bn[u] = at32(bin1, min(k[u], J.N1 - 1u));
 #pragma unroll
       for (uint32_t u = 0; u < kShufU; ++u)
         if (m[u] < J.N1) nb_st<NBL>(S, m[u], (uint16_t)bn[u]);
@@ -394,15 +403,13 @@ __device__ __forceinline__ void build_rows(const DevJob &J, const LdsLayout &Lo,
   } else {
     for (uint32_t k0 = tid; k0 < J.N1; k0 += NT * kU) {
       uint32_t m[kU], bn[kU];
+      /* clamped loads: under a condition each load is a basic block of its
+       * own, and its wait comes before the next one */
 #pragma unroll
       for (uint32_t u = 0; u < kU; ++u) {
-        const uint32_t k = k0 + u * NT;
-        m[u] = 0u;
-        bn[u] = 0u;
-        if (k < J.N1) {
-          m[u] = i1 ? i1[k] : k;
-          bn[u] = bin1[k];
-        }
+        const uint32_t k = min(k0 + u * NT, J.N1 - 1u);
+        m[u] = i1 ? at32(i1, k) : k;
+        bn[u] = at32(bin1, k);
       }
 #pragma unroll
       for (uint32_t u = 0; u < kU; ++u) {
@@ -448,9 +455,8 @@ __device__ __forceinline__ void build_rows(const DevJob &J, const LdsLayout &Lo,
       int32_t jm[kShufU];
 #pragma unroll
       for (uint32_t u = 0; u < kShufU; ++u) {
-        const bool in = q[u] < J.N2;
-        b[u] = in ? bin2[e[u]] : kBinNone;
-        jm[u] = (in && !J.dup) ? join[q[u]] : -1;
+        b[u] = at32(bin2, min(e[u], J.N2 - 1u));
+        jm[u] = at32(join, min(q[u], J.N2 - 1u));
       }
 #pragma unroll
       for (uint32_t u = 0; u < kShufU; ++u)
@@ -462,16 +468,12 @@ __device__ __forceinline__ void build_rows(const DevJob &J, const LdsLayout &Lo,
       int32_t jm[kU];
 #pragma unroll
       for (uint32_t u = 0; u < kU; ++u) {
-        const uint32_t e = e0 + u * NT;
-        q[u] = kNone;
-        b[u] = kBinNone;
-        if (e < J.N2) {
-          q[u] = i2 ? i2[e] : e;
-          b[u] = bin2[e];
-        }
+        const uint32_t e = min(e0 + u * NT, J.N2 - 1u);
+        q[u] = i2 ? at32(i2, e) : e;
+        b[u] = at32(bin2, e);
       }
 #pragma unroll
-      for (uint32_t u = 0; u < kU; ++u) jm[u] = (q[u] < J.N2 && !J.dup) ? join[q[u]] : -1;
+      for (uint32_t u = 0; u < kU; ++u) jm[u] = at32(join, min(q[u], J.N2 - 1u));
 #pragma unroll
       for (uint32_t u = 0; u < kU; ++u) {
         const uint32_t e = e0 + u * NT;
