@@ -221,9 +221,16 @@ int upload_job(dto_job *j) {
     j->arena = nullptr;
   }
   j->resident = false;
-  HIP_TRY(hipMalloc(&j->arena, j->image.size()));
+  /* after the tables: the error word, the records of a small run and one
+   * pair of index arrays, so that calls need no allocation of their own and
+   * one copy brings the error word and the records back */
+  const size_t tables = j->image.size();
+  j->image.resize(tables + kErrBytes, 0);
+  HIP_TRY(hipMalloc(&j->arena, j->image.size() + kCallRecords * sizeof(dto_record) +
+                                   ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t)));
   HIP_TRY(hipMemcpy(j->arena, j->image.data(), j->image.size(), hipMemcpyHostToDevice));
   bind_job(j, (unsigned char *)j->arena);
+  j->d_err = (int *)((unsigned char *)j->arena + tables);
   std::vector<unsigned char>().swap(j->image); /* the device copy is the job's now */
   /* global pair staging for layouts whose pairs do not fit in LDS */
   if (j->ws) {
@@ -294,29 +301,76 @@ static int check_err_flag(dto_job *j) {
   return DTO_OK;
 }
 
-/* explicit permutations must be permutations of [0, len) */
-static int validate_perms(const uint32_t *idx, uint64_t P, uint64_t len) {
-  if (!idx) return DTO_OK;
-  std::vector<uint64_t> stamp(len, 0);
-  for (uint64_t p = 0; p < P; ++p) {
-    const uint32_t *row = idx + p * len;
-    for (uint64_t k = 0; k < len; ++k) {
-      uint32_t v = row[k];
-      if (v >= len || stamp[v] == p + 1)
-        return fail(DTO_ERR_BAD_PERMUTATION, "permutation " + std::to_string(p) + " is not a permutation of [0, " +
-                                                 std::to_string(len) + ")");
-      stamp[v] = p + 1;
-    }
-  }
-  return DTO_OK;
-}
-
 struct DevBuf {
   void *p = nullptr;
   ~DevBuf() {
     if (p) (void)hipFree(p);
   }
 };
+
+/* Device room for one call's records (and, for a single explicit pair, its
+ * index arrays): the job's own where it is free and large enough, else
+ * allocated for the call. */
+struct CallRoom {
+  dto_job *j;
+  std::unique_lock<std::mutex> own;
+  DevBuf tmp;
+  dto_record *rec = nullptr;
+  uint32_t *idx = nullptr;
+  size_t records = 0;
+  explicit CallRoom(dto_job *job) : j(job) {}
+  int open(size_t n, bool with_idx) {
+    records = n;
+    const size_t rec_b = n * sizeof(dto_record);
+    if (j->arena && n <= kCallRecords) {
+      own = std::unique_lock<std::mutex>(j->call_mu, std::try_to_lock);
+      if (own.owns_lock()) {
+        rec = (dto_record *)((unsigned char *)j->d_err + kErrBytes);
+        idx = (uint32_t *)(rec + kCallRecords);
+        return DTO_OK;
+      }
+    }
+    const size_t idx_b = with_idx ? ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t) : 0;
+    HIP_TRY(hipMalloc(&tmp.p, rec_b + idx_b));
+    rec = (dto_record *)tmp.p;
+    idx = (uint32_t *)((unsigned char *)tmp.p + rec_b);
+    return DTO_OK;
+  }
+  /* Waits for the launches of this call and brings its records back. */
+  int fetch(std::vector<unsigned char> &buf, const dto_record **out) {
+    const size_t rec_b = records * sizeof(dto_record);
+    buf.resize(kErrBytes + rec_b);
+    *out = (const dto_record *)(buf.data() + kErrBytes);
+    if (!own.owns_lock()) {
+      HIP_TRY(hipMemcpy(buf.data() + kErrBytes, rec, rec_b, hipMemcpyDeviceToHost));
+      return check_err_flag(j);
+    }
+    HIP_TRY(hipMemcpy(buf.data(), j->d_err, kErrBytes + rec_b, hipMemcpyDeviceToHost));
+    int err;
+    memcpy(&err, buf.data(), sizeof err);
+    return err ? check_err_flag(j) : DTO_OK;
+  }
+};
+
+/* explicit permutations must be permutations of [0, len) */
+static int validate_perms(const uint32_t *idx, uint64_t P, uint64_t len) {
+  if (!idx) return DTO_OK;
+  std::vector<uint8_t> stamp(len, 0); /* the last of 255 rounds of rows that held the value */
+  for (uint64_t p = 0; p < P; ++p) {
+    const uint32_t *row = idx + p * len;
+    const uint8_t mark = (uint8_t)(p % 255u + 1u);
+    if (p && mark == 1u) std::fill(stamp.begin(), stamp.end(), (uint8_t)0);
+    for (uint64_t k = 0; k < len; ++k) {
+      uint32_t v = row[k];
+      if (v >= len || stamp[v] == mark)
+        return fail(DTO_ERR_BAD_PERMUTATION, "permutation " + std::to_string(p) + " is not a permutation of [0, " +
+                                                 std::to_string(len) + ")");
+      stamp[v] = mark;
+    }
+  }
+  return DTO_OK;
+}
+
 
 /* ------------------------------------------------------------------ */
 /* C ABI                                                                  */
@@ -584,23 +638,27 @@ int dto_optimize(dto_job *job, const uint32_t *idx1, const uint32_t *idx2, uint3
   int rc;
   if ((rc = ensure_resident(job))) return rc;
   if ((rc = validate_perms(idx1, 1, job->dev.N1)) || (rc = validate_perms(idx2, 1, job->dev.N2))) return rc;
-  DevBuf di, dr;
   const size_t n1 = job->dev.N1, n2 = job->dev.N2;
-  HIP_TRY(hipMalloc(&di.p, (n1 + n2 + 2) * 4));
-  HIP_TRY(hipMalloc(&dr.p, sizeof(dto_record)));
-  uint32_t *d1 = nullptr, *d2 = nullptr;
-  if (idx1) {
-    d1 = (uint32_t *)di.p;
+  CallRoom room(job);
+  if ((rc = room.open(1, true))) return rc;
+  uint32_t *d1 = idx1 ? room.idx : nullptr, *d2 = idx2 ? room.idx + n1 : nullptr;
+  if (idx1 && idx2) {
+    std::vector<uint32_t> both(n1 + n2);
+    memcpy(both.data(), idx1, n1 * 4);
+    memcpy(both.data() + n1, idx2, n2 * 4);
+    HIP_TRY(hipMemcpy(d1, both.data(), (n1 + n2) * 4, hipMemcpyHostToDevice));
+  } else if (idx1) {
     HIP_TRY(hipMemcpy(d1, idx1, n1 * 4, hipMemcpyHostToDevice));
-  }
-  if (idx2) {
-    d2 = (uint32_t *)di.p + n1 + 1;
+  } else if (idx2) {
     HIP_TRY(hipMemcpy(d2, idx2, n2 * 4, hipMemcpyHostToDevice));
   }
   int32_t permuted = (idx1 || idx2) ? 1 : 0;
-  if ((rc = launch_perms(job, mode, true, d1, d2, 1, 0, 0, 0, permuted, (dto_record *)dr.p, 0))) return rc;
-  HIP_TRY(hipMemcpy(out, dr.p, sizeof(dto_record), hipMemcpyDeviceToHost));
-  return check_err_flag(job);
+  if ((rc = launch_perms(job, mode, true, d1, d2, 1, 0, 0, 0, permuted, room.rec, 0))) return rc;
+  std::vector<unsigned char> buf;
+  const dto_record *rec = nullptr;
+  if ((rc = room.fetch(buf, &rec))) return rc;
+  *out = *rec;
+  return DTO_OK;
 }
 
 int dto_process_threshold_pairs(dto_job *job, const uint32_t *idx1, const uint32_t *idx2, dto_record *out) {
@@ -651,9 +709,9 @@ int dto_run(dto_job *job, uint64_t n_perm, uint64_t seed, const uint32_t *idx1, 
   if ((rc = ensure_resident(job))) return rc;
   const uint64_t n1 = job->dev.N1, n2 = job->dev.N2;
   if ((rc = validate_perms(idx1, n_perm, n1)) || (rc = validate_perms(idx2, n_perm, n2))) return rc;
-  DevBuf dr;
-  HIP_TRY(hipMalloc(&dr.p, (n_perm + 1) * sizeof(dto_record)));
-  dto_record *d_rec = (dto_record *)dr.p;
+  CallRoom room(job);
+  if ((rc = room.open(n_perm + 1, false))) return rc;
+  dto_record *d_rec = room.rec;
   /* task 0: unpermuted (main.rs:122-125); with drawn permutations it joins
    * their launch, where it costs no workgroup's latency of its own */
   const uint32_t lead = mode == DTO_MODE_SCREENED && n_perm && !idx1 ? 1 : 0;
@@ -678,11 +736,11 @@ int dto_run(dto_job *job, uint64_t n_perm, uint64_t seed, const uint32_t *idx1, 
         return rc;
     }
   }
-  std::vector<dto_record> rec(n_perm + 1);
-  HIP_TRY(hipMemcpy(rec.data(), d_rec, (n_perm + 1) * sizeof(dto_record), hipMemcpyDeviceToHost));
-  if ((rc = check_err_flag(job))) return rc;
-  if (perm_out && n_perm) memcpy(perm_out, rec.data() + 1, n_perm * sizeof(dto_record));
-  return dto_empirical_pvalue(&rec[0], rec.data() + 1, n_perm, result);
+  std::vector<unsigned char> buf;
+  const dto_record *rec = nullptr;
+  if ((rc = room.fetch(buf, &rec))) return rc;
+  if (perm_out && n_perm) memcpy(perm_out, rec + 1, n_perm * sizeof(dto_record));
+  return dto_empirical_pvalue(&rec[0], rec + 1, n_perm, result);
 }
 
 int dto_result_json(const dto_result *result, char *buf, size_t cap) {

@@ -47,6 +47,9 @@ void cut_levels(const HostJob &h, DevJob &d);
 }  // namespace dto
 
 constexpr uint32_t kCounterRing = 256;
+/* A resident job's room for small calls (upload_job): bytes of the error
+ * word's block, and records after it (a run of 1,000 permutations). */
+constexpr size_t kErrBytes = 256, kCallRecords = 1025;
 
 /* Byte offsets of a job's tables inside its device arena. */
 struct ArenaOffsets {
@@ -84,6 +87,7 @@ struct dto_job {
   hipEvent_t ws_ev = nullptr;
   bool ws_used = false;
   std::mutex ws_mu;
+  std::mutex call_mu; /* the arena's call room is in use */
 };
 /* Tables, layouts and arena image of a job on the current device (no device
  * memory); then either its own arena (upload_job) or a caller's region
