@@ -182,7 +182,11 @@ static __global__ __launch_bounds__(256) void k_grid_pvalues(DevJob J, const uin
   __syncthreads();
   const uint32_t lane = lane_id(), w = wave_id();
   const uint64_t cells = (uint64_t)J.T1 * J.T2;
-  for (uint64_t c0 = ((uint64_t)blockIdx.x * 4u + w) * 64u; c0 < cells; c0 += (uint64_t)gridDim.x * 256u) {
+  /* from the last cells on: the long tails are in the later rows, and would
+   * otherwise run on when the rest is done */
+  const uint64_t batches = (cells + 63u) / 64u;
+  for (uint64_t q = (uint64_t)blockIdx.x * 4u + w; q < batches; q += (uint64_t)gridDim.x * 4u) {
+    const uint64_t c0 = (batches - 1u - q) * 64u;
     const uint64_t c = c0 + lane;
     if (c < cells) {
       const uint32_t i = (uint32_t)(c / J.T2), j = (uint32_t)(c % J.T2);
