@@ -63,15 +63,16 @@ __device__ __forceinline__ double log_term(const DevJob &J, uint32_t K, uint32_t
 
 /* The cut tables: out[(((level * T1 + i) * segs + s) * kCutWords + u) * 64 +
  * lane] packs the cuts of columns 2 w and 2 w + 1, w = kCutSpan s + kCutWords
- * lane + u.  A cell is dropped when k <= its cut.  One thread per cell finds
- * the largest k0 above the mode with P(X = k0) >= e^(L - 7), L the lowest
- * level, by bisection, then adds terms downwards from k0 in FP32: at every k
- * the sum is a lower bound of P(X >= k) up to its rounding (each term's ratio
- * has a relative error below 4 * 2^-24; at 2,000 terms under 1e-3 together),
- * so P(X >= k) > e^l is certain for each level l once the sum exceeds 1.01
- * e^l, and for every smaller k too.  A tail that never gets there keeps the
- * cut max(0, K + n - N), the largest k with P(X >= k) = 1, which is also
- * level 0's.  Columns past T2 get 0xFFFF: never listed. */
+ * lane + u.  A cell is dropped when k <= its cut.  One thread per cell.  For
+ * the low levels the cut is the largest k found with P(X = k) alone above the
+ * level.  From there it adds terms downwards in FP32: at every k the sum is a
+ * lower bound of P(X >= k) up to its rounding (each term's ratio has a
+ * relative error below 4 * 2^-24, and above populations of 2^24 the counts'
+ * own rounding adds under 0.6 % at the longest accepted lists), so P(X >= k)
+ * > e^l is certain once the sum exceeds 1.01 e^l, and for every smaller k
+ * too.  A tail that never gets there keeps the cut max(0, K + n - N), the
+ * largest k with P(X >= k) = 1, which is also level 0's.  Columns past T2 get
+ * 0xFFFF: never listed. */
 static __global__ __launch_bounds__(256) void k_cut_table(DevJob J, uint16_t *__restrict__ out) {
   const uint32_t cols = 2u * kCutSpan * J.cut_segs;
   const uint64_t per_level = (uint64_t)J.T1 * cols;
@@ -86,33 +87,45 @@ static __global__ __launch_bounds__(256) void k_cut_table(DevJob J, uint16_t *__
     }
     const uint32_t N = J.N, K = J.K[i], n = J.n[j];
     const uint32_t lo = K + n > N ? K + n - N : 0u, hi = K < n ? K : n;
-    const double low = (double)J.cut_level[kCutLevels - 1];
-    /* largest k >= mode with log P(X = k) >= low - 7 (terms fall above the mode) */
-    uint32_t k = (uint32_t)(((double)K + 1.0) * ((double)n + 1.0) / ((double)N + 2.0));
-    k = k < lo ? lo : (k > hi ? hi : k);
-    uint32_t b = hi;
-    while (k < b) {
-      const uint32_t m = b - (b - k) / 2u;
-      if (log_term(J, K, n, m) >= low - 7.0)
-        k = m;
-      else
-        b = m - 1u;
-    }
-    float t = __expf((float)(log_term(J, K, n, k) - low)), S = t;
-    uint32_t l = kCutLevels - 1u;
-    float th = 1.01f;
-    for (; k > lo; --k) {
-      while (S > th) {
-        o[l * per_level] = (uint16_t)k;
-        --l;
-        th = l ? 1.01f * __expf(J.cut_level[l] - (float)low) : __builtin_inff();
+    uint32_t mode = (uint32_t)(((double)K + 1.0) * ((double)n + 1.0) / ((double)N + 2.0));
+    mode = mode < lo ? lo : (mode > hi ? hi : mode);
+    /* the low levels, by the first term alone: Newton steps down from the
+     * largest k (log P(X = k) is concave, so a step rounded down stays on the
+     * far side of the level until the last ones) */
+    uint32_t k = hi, l = kCutLevels - 1u;
+    double x = log_term(J, K, n, k);
+    for (; l >= kCutDeep; --l) {
+      const double level = (double)J.cut_level[l] + 0.01;
+      while (x < level && k > mode) {
+        const float s = __logf((float)k * (float)((N - K) - (n - k)) / ((float)(K - k + 1u) * (float)(n - k + 1u)));
+        const float d = s > 1e-3f ? fminf((float)(level - x) / s, 1e9f) : 1.f;
+        const uint32_t step = d > 1.f ? (uint32_t)d : 1u;
+        k -= step < k - mode ? step : k - mode;
+        x = log_term(J, K, n, k);
       }
-      if (l == 0u) break;
-      /* t_{k-1} / t_k */
-      const float num = (float)k * (float)((N - K) - (n - k));
-      const float den = (float)(K - k + 1u) * (float)(n - k + 1u);
-      t *= num * __builtin_amdgcn_rcpf(den);
-      S += t;
+      if (x < level) break;
+      o[l * per_level] = (uint16_t)k;
+    }
+    if (l < kCutDeep) {
+      /* the others, by the sum from here down, in units of the first term */
+      const float off = (float)x;
+      float t = 1.f, S = 1.f, th = 1.01f * __expf(J.cut_level[l] - off);
+      /* t_{k-1} / t_k = k (N - K - n + k) / ((K - k + 1) (n - k + 1)) */
+      float f0 = (float)k, f1 = (float)((N - K) - (n - k)), f2 = (float)(K - k + 1u), f3 = (float)(n - k + 1u);
+      for (; k > lo; --k) {
+        while (S > th) {
+          o[l * per_level] = (uint16_t)k;
+          --l;
+          th = l ? 1.01f * __expf(J.cut_level[l] - off) : __builtin_inff();
+        }
+        if (l == 0u) break;
+        t *= (f0 * f1) * __builtin_amdgcn_rcpf(f2 * f3);
+        S += t;
+        f0 -= 1.f;
+        f1 -= 1.f;
+        f2 += 1.f;
+        f3 += 1.f;
+      }
     }
     for (uint32_t v = 0; v <= l; ++v) o[v * per_level] = (uint16_t)lo;
   }
@@ -321,7 +334,7 @@ __device__ __forceinline__ void flush_cut(const DevJob &J, const Lds &S, uint2 *
 /* First row of wave w's block: rows are split so that the sum of rows
  * (kRowPairs pairs' worth of work each) and pairs is about equal per wave.
  * The lanes probe 64 rows at a time. */
-constexpr uint32_t kRowPairs = 192;
+constexpr uint32_t kRowPairs = 512;
 __device__ __forceinline__ uint32_t block_row(const uint32_t *rowstart, uint32_t T1, uint32_t w, uint32_t W) {
   if (w == 0u) return 0u;
   if (w >= W) return T1;

@@ -15,8 +15,9 @@ namespace dto {
 constexpr uint32_t kBinNone = 0xFFFFu; /* (a,b) pair outside the grid */
 
 /* Levels of the cut tables, and the one a permutation's sweep starts with. */
-constexpr uint32_t kCutLevels = 12;
+constexpr uint32_t kCutLevels = 14;
 constexpr uint32_t kCutStart = 5;
+constexpr uint32_t kCutDeep = 9; /* from this one on, cuts come from the first term alone */
 
 struct DevJob {
   uint32_t N;        /* population size */

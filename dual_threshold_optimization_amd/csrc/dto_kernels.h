@@ -5,24 +5,24 @@
  * (src/dto/process_threshold_pairs.rs:71-131, src/dto/optimize_main.rs:53-118),
  * and the std::thread permutation loop (src/run/single_node.rs:83-137).
  *
- * One workgroup owns one permutation at a time (grid-stride over
- * permutations; the per-job tables stay in LDS across them):
+ * One workgroup owns one permutation at a time.  This file holds what the
+ * kernels share (the build of a permutation's row-sorted pairs, the exact
+ * and bracket tiers, the tie-break) and the first-term screen of serving
+ * slices; dto_cut.h holds the screened kernels of jobs with cut tables,
+ * dto_plain.h the plain mode and the debug grid.
  *   A  scatter: list1 feature m takes the bin of the position it lands on,
  *      nb[idx1[k]] = bin1[k]                                  (LDS, u16)
  *   B  pairs: list2 position e holds entry q = idx2[e]; its list1 partner's
  *      bin a = nb[join[q]], its own bin b = bin2[e]; counting sort of the
  *      pairs by a (row) into nb                                 (LDS)
- *   C  per-wave column histograms of row blocks, prefix over waves
- *   D  each wave sweeps its rows: add the row's pairs into its running
+ *   D  each wave sweeps its rows: add the rows' pairs into its running
  *      column counts, wave prefix scan -> exact overlap k(i, j) for the row,
- *      then per cell either
- *        PLAIN:    the exact FP64 statrs tail (dto_tail_exact), or
- *        SCREENED: an FP32 log-space bound of the tail from the LDS table
- *                  H(x) = ln x! - x (ln N - 1); cells that cannot reach the
- *                  minimum are dropped, p == 0 and p == 1 classes are exact.
- *   E  SCREENED only: reverse sweep over rows that can hold the minimum;
- *      surviving cells are evaluated exactly in FP64 (bit-identical to the
- *      reference) and reduced with the reference tie-break.
+ *      then per cell an FP32 log-space bound of the tail from the LDS table
+ *      H(x) = ln x! - x (ln N - 1); cells that cannot reach the minimum are
+ *      dropped, p == 0 and p == 1 classes are exact.
+ *   E  reverse sweep over rows that can hold the minimum; surviving cells
+ *      are evaluated exactly in FP64 (bit-identical to the reference) and
+ *      reduced with the reference tie-break.
  * No MFMA: nothing here is a dense contraction.
  */
 #pragma once
@@ -318,15 +318,17 @@ __device__ __forceinline__ void shuffle_chunk(const Shuffle &s, uint32_t *wsum, 
                                               uint32_t *rk, uint32_t *v) {
   constexpr uint32_t W = NT / 64;
   const uint32_t lane = lane_id(), w = wave_id();
-  const uint32_t p0 = base + w * (64u * kShufU) + lane;
+  const uint32_t p0 = base + w * (64u * kShufU);
   uint32_t cnt = 0u; /* elements below n in the wave's earlier steps */
 #pragma unroll
   for (uint32_t u = 0; u < kShufU; ++u) {
-    const uint32_t p = p0 + 64u * u;
+    /* 64 consecutive elements from a multiple of 64 share their high part (2^pa
+     * >= 64), whose first mix is then scalar work */
+    const uint32_t q = p0 + 64u * u, p = q + lane;
     if (s.ident)
       v[u] = min(p, s.n);
     else
-      v[u] = p < s.dom ? feistel_once(s, p) : s.n;
+      v[u] = p < s.dom ? feistel_pair(s, (q & s.amask) + lane, q >> s.pa) : s.n;
     const uint64_t m = __ballot(v[u] < s.n);
     rk[u] = cnt + mask_lt(m);
     cnt += (uint32_t)__popcll(m);

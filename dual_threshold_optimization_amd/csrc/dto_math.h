@@ -287,9 +287,8 @@ DTO_HD uint32_t feistel_mix(uint32_t v, uint32_t key) {
   return h ^ (key >> 24);
 }
 
-/* F(v): the Feistel bijection of [0, dom). */
-DTO_HD uint32_t feistel_once(const Shuffle &s, uint32_t v) {
-  uint32_t L = v & s.amask, R = v >> s.pa;
+/* F(v), v = R * 2^pa + L: the Feistel bijection of [0, dom). */
+DTO_HD uint32_t feistel_pair(const Shuffle &s, uint32_t L, uint32_t R) {
 #pragma unroll
   for (int r = 0; r < DTO_FEISTEL_ROUNDS; ++r) {
     if ((r & 1) == 0) {
@@ -303,6 +302,7 @@ DTO_HD uint32_t feistel_once(const Shuffle &s, uint32_t v) {
   }
   return (R << s.pa) | L;
 }
+DTO_HD uint32_t feistel_once(const Shuffle &s, uint32_t v) { return feistel_pair(s, v & s.amask, v >> s.pa); }
 
 /* The whole permutation (host): out[k] = idx[k], k < n. */
 static inline void shuffle_fill(const Shuffle &s, uint32_t *out) {
