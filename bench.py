@@ -52,8 +52,8 @@ def parse():
     p.add_argument("--cli-runs", type=int, default=10, help="timed runs of the CLI on the README lists")
     p.add_argument("--only", choices=["all", "headline", "calibrate-copy"], default="all")
     p.add_argument("--no-cpu", action="store_true")
-    p.add_argument("--traffic-file", default=os.path.join(ROOT, "profiles", "k_optimize_genome_20k_pmc.txt"))
-    p.add_argument("--sq-file", default=os.path.join(ROOT, "profiles", "k_optimize_genome_20k_sq_counters.txt"))
+    p.add_argument("--traffic-file", default=os.path.join(ROOT, "profiles", "k_cut_genome_20k_pmc.txt"))
+    p.add_argument("--sq-file", default=os.path.join(ROOT, "profiles", "k_cut_genome_20k_sq_counters.txt"))
     return p.parse_args()
 
 
@@ -172,10 +172,9 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": read_traffic(args.traffic_file),
                 "valu_issue_frac": valu_frac,
-                "valu_issue_basis": "SQ_INSTS_VALU per launch (profiles/k_optimize_genome_20k_sq_counters.txt) / "
+                "valu_issue_basis": "SQ_INSTS_VALU per launch (profiles/k_cut_genome_20k_sq_counters.txt) / "
                                     "(live kernel time x 256 CUs x 4 SIMDs x 2.4 GHz / 4)",
-                "kernel": "k_optimize<512 threads, explicit permutations, H table in LDS, screened, pairs in LDS, "
-                          "column constants in registers, bins in LDS>",
+                "kernel": "k_cut<1024 threads, explicit permutations, pairs in registers, join and bins in LDS>",
                 "kernel_ms": round(kern_ms, 4),
                 "algorithmic_bytes_per_launch": bytes_per_launch}
 
@@ -186,7 +185,7 @@ def main():
               "config": {"workload": "genome_20k: lists 22,000 features, background 20,000 (N=20,000 after drop), "
                                      "600 planted, 10%% ties, reference thresholds (T=%dx%d), unpermuted + %d explicit "
                                      "permutations per step" % (job.n_thresholds1, job.n_thresholds2, P),
-                         "mode": "screened (FP32 log-space screen + exact FP64 recheck)"},
+                         "mode": "screened (critical-count screen + exact FP64 recheck)"},
               "roofline": roofline}
     if args.only == "headline":
         print(json.dumps(result))

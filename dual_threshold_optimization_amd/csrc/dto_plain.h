@@ -57,7 +57,8 @@ __device__ __forceinline__ double tail_exact_wide(const double *LF, uint32_t N, 
  * writes the record.  The lanes of a wave take 128 neighbouring columns at a
  * time, whose tails are of similar length.  Items come from a device counter
  * (zeroed before the launch); every workgroup exits once it passes n_perm *
- * parts. */
+ * parts.  49 tasks at N = 6,000: 2.45 ms, 25.7 ms with a workgroup a task,
+ * ten neighbouring columns a lane and one term at a time. */
 template <int NT, bool EXPLICIT, bool PL>
 __global__ __launch_bounds__(NT) void k_plain(DevJob J, LdsLayout Lo, const uint32_t *__restrict__ idx1,
                                               const uint32_t *__restrict__ idx2, uint64_t n_perm, uint64_t perm_base,
@@ -142,7 +143,8 @@ static __global__ __launch_bounds__(64) void k_plain_reduce(DevJob J, const Best
 
 /* Overlap counts of every cell of one permutation: the workgroups build the
  * rows each for itself, and wave s of all takes rows s, s + waves, ...
- * (a launch of one workgroup swept every row after the other). */
+ * (a launch of one workgroup swept every row after the other: with 64, 45 us
+ * for the 599 rows at N = 20,000, most of it the build). */
 template <int NT, bool PL>
 __global__ __launch_bounds__(NT) void k_grid_counts(DevJob J, LdsLayout Lo, const uint32_t *__restrict__ idx1,
                                                     const uint32_t *__restrict__ idx2, uint32_t *__restrict__ kout,
