@@ -9,11 +9,14 @@
 
 namespace dto {
 
-/* dto_tail_exact with kTailUnroll terms in flight: their table loads and exps
- * are independent, and only the additions, made in the same ascending order
- * with the same early exit, are serial, so the sum is bit-identical.  One
- * term at a time waits for four table reads and an exp per addition. */
-constexpr uint32_t kTailUnroll = 4;
+/* dto_tail_exact with U terms in flight: their table loads and exps are
+ * independent, and only the additions, made in the same ascending order with
+ * the same early exit, are serial, so the sum is bit-identical.  One term at a
+ * time waits for four table reads and an exp per addition.  Four where the
+ * tasks fill the GPU (49 plain tasks at N = 6,000: 2.45 ms, 2.87 with eight);
+ * eight for the one grid of a call, which waits for its longest tails (599 x
+ * 599 records: 247 us, 256 with four). */
+template <uint32_t U>
 __device__ __forceinline__ double tail_exact_wide(const double *LF, uint32_t N, uint32_t K, uint32_t n, uint32_t k,
                                                   double d, const uint64_t *tab) {
   if (k == 0) return 1.0;
@@ -23,19 +26,19 @@ __device__ __forceinline__ double tail_exact_wide(const double *LF, uint32_t N, 
   const double lfK = LF[K], lfNK = LF[N - K];
   const uint32_t NK = N - K;
   double acc = 0.0;
-  for (uint32_t i0 = k; i0 <= mx; i0 += kTailUnroll) {
-    double t[kTailUnroll];
+  for (uint32_t i0 = k; i0 <= mx; i0 += U) {
+    double t[U];
 #pragma unroll
-    for (uint32_t u = 0; u < kTailUnroll; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
       const uint32_t i = min(i0 + u, mx);
       const double lb1 = (lfK - LF[i]) - LF[K - i];
       const double lb2 = (lfNK - LF[n - i]) - LF[NK - (n - i)];
       t[u] = (lb1 + lb2) - d;
     }
 #pragma unroll
-    for (uint32_t u = 0; u < kTailUnroll; ++u) t[u] = dto_exp(t[u], tab);
+    for (uint32_t u = 0; u < U; ++u) t[u] = dto_exp(t[u], tab);
 #pragma unroll
-    for (uint32_t u = 0; u < kTailUnroll; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
       const uint32_t i = i0 + u;
       if (i > mx) return acc;
       acc = acc + t[u];
@@ -108,7 +111,7 @@ __global__ __launch_bounds__(NT) void k_plain(DevJob J, LdsLayout Lo, const uint
         for (uint32_t h = 0; h < 2; ++h) {
           const uint32_t j = 2u * wi + h;
           k += h ? x >> 16 : x & 0xFFFFu;
-          if (j < T2) take_better(xb, tail_exact_wide(J.LF, J.N, K, S.coln[j], k, J.D[j], S.tab), k, (i << 16) | j);
+          if (j < T2) take_better(xb, tail_exact_wide<4>(J.LF, J.N, K, S.coln[j], k, J.D[j], S.tab), k, (i << 16) | j);
         }
       }
     }
@@ -193,7 +196,7 @@ static __global__ __launch_bounds__(256) void k_grid_pvalues(DevJob J, const uin
     if (c < cells) {
       const uint32_t i = (uint32_t)(c / J.T2), j = (uint32_t)(c % J.T2);
       const uint32_t k = kin[c];
-      const double p = tail_exact_wide(J.LF, J.N, J.K[i], J.n[j], k, J.D[j], tab);
+      const double p = tail_exact_wide<8>(J.LF, J.N, J.K[i], J.n[j], k, J.D[j], tab);
       write_record(J, BestKey{p, k, (i << 16) | j, 0u, 0u}, permuted, &stage[w][lane], nullptr);
     }
     wave_sync();
