@@ -1698,6 +1698,10 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchJob *__restrict__ jobs,
         b = optimize_perm<NT, false, HLDS, PL, REGCOLS, NBL>(B.J, B.lo, S, nullptr, nullptr, s1, s2, err, st, gpairs);
       }
       if (threadIdx.x == 0) write_record(B.J, b, t == 0 ? 0 : 1, B.out + t, err);
+      /* keeps thread 0's block apart from the next claim's: joined, the other
+       * lanes of its wave could go round the loop, past the claim's barrier,
+       * ahead of thread 0 */
+      wave_sync();
     }
   }
 }
