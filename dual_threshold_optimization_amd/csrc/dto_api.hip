@@ -216,32 +216,29 @@ int upload_job(dto_job *j) {
   if (rc) return rc;
   DevProps pr;
   if ((rc = device_props(j->device, &pr))) return rc;
-  if (j->arena) {
-    (void)hipFree(j->arena);
-    j->arena = nullptr;
-  }
+  if (j->arena) (void)hipFree(j->arena);
+  if (j->ws) (void)hipFree(j->ws);
+  j->arena = nullptr;
+  j->ws = nullptr;
   j->resident = false;
+  /* global pair staging for layouts whose pairs do not fit in LDS; before the
+   * job is resident, so that no launch finds it missing */
+  j->ws_slots = (uint32_t)pr.cus * 4u;
+  if (!j->lo_plain.pairs_in_lds || !j->lo_cut.pairs_in_lds) {
+    HIP_TRY(j->alloc((void **)&j->ws, (size_t)j->ws_slots * std::max<uint32_t>(j->dev.N2, 1) * sizeof(uint16_t)));
+    if (!j->ws_ev) HIP_TRY(hipEventCreateWithFlags(&j->ws_ev, hipEventDisableTiming));
+  }
   /* after the tables: the error word, the records of a small run and one
    * pair of index arrays, so that calls need no allocation of their own and
    * one copy brings the error word and the records back */
   const size_t tables = j->image.size();
   j->image.resize(tables + kErrBytes, 0);
-  HIP_TRY(hipMalloc(&j->arena, j->image.size() + kCallRecords * sizeof(dto_record) +
-                                   ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t)));
+  HIP_TRY(j->alloc(&j->arena, j->image.size() + kCallRecords * sizeof(dto_record) +
+                                  ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t)));
   HIP_TRY(hipMemcpy(j->arena, j->image.data(), j->image.size(), hipMemcpyHostToDevice));
   bind_job(j, (unsigned char *)j->arena);
   j->d_err = (int *)((unsigned char *)j->arena + tables);
   std::vector<unsigned char>().swap(j->image); /* the device copy is the job's now */
-  /* global pair staging for layouts whose pairs do not fit in LDS */
-  if (j->ws) {
-    (void)hipFree(j->ws);
-    j->ws = nullptr;
-  }
-  j->ws_slots = (uint32_t)pr.cus * 4u;
-  if (!j->lo_plain.pairs_in_lds || !j->lo_cut.pairs_in_lds) {
-    HIP_TRY(hipMalloc(&j->ws, (size_t)j->ws_slots * std::max<uint32_t>(j->dev.N2, 1) * sizeof(uint16_t)));
-    if (!j->ws_ev) HIP_TRY(hipEventCreateWithFlags(&j->ws_ev, hipEventDisableTiming));
-  }
   return ensure_cut(j, 0);
 }
 
@@ -516,6 +513,14 @@ int dto_internal_stats(dto_job *job, uint64_t *out, int reset) {
   HIP_TRY(hipDeviceSynchronize());
   HIP_TRY(hipMemcpy(out, job->dev.stats, 16 * sizeof(uint64_t), hipMemcpyDeviceToHost));
   if (reset) HIP_TRY(hipMemset(job->dev.stats, 0, 16 * sizeof(uint64_t)));
+  return DTO_OK;
+}
+
+/* test hook (not in dto.h): the n-th device allocation of the job from now on
+ * fails (0: none does) */
+int dto_internal_fail_alloc(dto_job *job, uint32_t n) {
+  if (!job) return fail(DTO_ERR_INVALID_ARGUMENT, "null pointer");
+  job->fail_alloc = n;
   return DTO_OK;
 }
 

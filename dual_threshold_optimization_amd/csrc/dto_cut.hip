@@ -96,7 +96,7 @@ int dto::ensure_cut(dto_job *j, hipStream_t st) {
   const size_t per_level = (size_t)j->dev.T1 * j->dev.cut_segs * 2u * kCutSpan;
   void *p = nullptr;
   /* the sweep loads one row's segment past the last */
-  HIP_TRY(hipMalloc(&p, (kCutLevels * per_level + 2u * kCutSpan) * sizeof(uint16_t)));
+  HIP_TRY(j->alloc(&p, (kCutLevels * per_level + 2u * kCutSpan) * sizeof(uint16_t)));
   const uint32_t grid = (uint32_t)std::min<size_t>((per_level + 255) / 256, 65536);
   hipLaunchKernelGGL(k_cut_table, dim3(grid), dim3(256), 0, st, j->dev, (uint16_t *)p);
   hipError_t e = hipGetLastError();

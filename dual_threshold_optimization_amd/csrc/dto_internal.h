@@ -88,6 +88,12 @@ struct dto_job {
   bool ws_used = false;
   std::mutex ws_mu;
   std::mutex call_mu; /* the arena's call room is in use */
+  std::atomic<uint32_t> fail_alloc{0}; /* test hook: the n-th allocation from now on fails */
+  /* The job's device allocations that later calls depend on. */
+  hipError_t alloc(void **p, size_t bytes) {
+    if (fail_alloc && --fail_alloc == 0) return hipErrorOutOfMemory;
+    return hipMalloc(p, bytes);
+  }
 };
 /* Tables, layouts and arena image of a job on the current device (no device
  * memory); then either its own arena (upload_job) or a caller's region
