@@ -56,6 +56,13 @@ struct ArenaOffsets {
   size_t bin1, bin2, join, joff, jpos, K, n, thr1, thr2, LF, D, H, A, B, err, ctr, stats;
 };
 
+/* The thread's stream-capture mode set to relaxed while in scope. */
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 /* A job: host tables plus their device copy (one HBM arena).  The arena is
  * the job's own allocation (`arena`), or, for a job created with
  * DTO_DEFER_UPLOAD and admitted by a server, a region of the server's pool
@@ -89,9 +96,13 @@ struct dto_job {
   std::mutex ws_mu;
   std::mutex call_mu; /* the arena's call room is in use */
   std::atomic<uint32_t> fail_alloc{0}; /* test hook: the n-th allocation from now on fails */
-  /* The job's device allocations that later calls depend on. */
+  /* The job's device allocations that later calls depend on.  Some are made
+   * by a launch: while any thread captures a stream in global mode, hipMalloc
+   * is refused to every thread (and may end that capture) unless the calling
+   * one is in relaxed mode. */
   hipError_t alloc(void **p, size_t bytes) {
     if (fail_alloc && --fail_alloc == 0) return hipErrorOutOfMemory;
+    RelaxedCapture relaxed;
     return hipMalloc(p, bytes);
   }
 };

@@ -18,22 +18,14 @@ using namespace dto;
  * launch on. */
 constexpr uint32_t kSplitTasks = 256, kSplitItems = 512;
 
-/* The launch's slot of the partial buffer, or NULL where there is none (under
- * a stream capture nothing can be allocated: the launch is not split). */
-static BestKey *partial_slot(dto_job *j, uint32_t slot, hipStream_t st) {
+/* The launch's slot of the partial buffer, or NULL where there is no memory
+ * for it (the launch is then not split). */
+static BestKey *partial_slot(dto_job *j, uint32_t slot) {
   std::lock_guard<std::mutex> g(j->cut_mu);
-  if (!j->partial) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    if (cs != hipStreamCaptureStatusNone) return nullptr;
-    if (hipMalloc(&j->partial, (size_t)kCounterRing * kSplitItems * sizeof(BestKey)) != hipSuccess) {
-      (void)hipGetLastError();
-      j->partial = nullptr;
-      return nullptr;
-    }
+  if (!j->partial && j->alloc(&j->partial, (size_t)kCounterRing * kSplitItems * sizeof(BestKey)) != hipSuccess) {
+    (void)hipGetLastError();
+    j->partial = nullptr;
+    return nullptr;
   }
   return (BestKey *)j->partial + (size_t)slot * kSplitItems;
 }
@@ -51,7 +43,7 @@ static hipError_t launch_t(dto_job *j, uint32_t max_grid, hipStream_t st, const 
   BestKey *partial = nullptr;
   if (n_perm <= kSplitTasks) {
     parts = std::min<uint32_t>(kSplitItems / (uint32_t)n_perm, (j->dev.T1 + kNT / 64 - 1) / (kNT / 64));
-    if (parts > 1 && !(partial = partial_slot(j, slot, st))) parts = 1;
+    if (parts > 1 && !(partial = partial_slot(j, slot))) parts = 1;
   }
   const uint32_t grid = (uint32_t)std::min<uint64_t>(n_perm * parts, max_grid);
   StagingOrder order(j, lo, st);
