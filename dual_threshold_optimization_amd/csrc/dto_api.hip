@@ -168,7 +168,7 @@ int prepare_job(dto_job *j) {
   o.A = put(buf, h.A32);
   o.B = put(buf, h.B32);
   o.err = put(buf, std::vector<int>(4, 0));
-  o.ctr = put(buf, std::vector<uint32_t>(kCounterRing, 0));
+  o.ctr = put(buf, std::vector<uint32_t>(kCounterSlots, 0));
   o.stats = put(buf, std::vector<unsigned long long>(16, 0));
   buf.resize((buf.size() + 255) & ~(size_t)255);
   j->arena_bytes = buf.size();
@@ -513,6 +513,15 @@ int dto_internal_stats(dto_job *job, uint64_t *out, int reset) {
   HIP_TRY(hipDeviceSynchronize());
   HIP_TRY(hipMemcpy(out, job->dev.stats, 16 * sizeof(uint64_t), hipMemcpyDeviceToHost));
   if (reset) HIP_TRY(hipMemset(job->dev.stats, 0, 16 * sizeof(uint64_t)));
+  return DTO_OK;
+}
+
+/* test hook (not in dto.h): the counter slots of n launches, captured[i] of
+ * them captured, in order */
+int dto_internal_launch_slots(const int32_t *captured, uint32_t n, uint32_t *out) {
+  if (!captured || !out) return fail(DTO_ERR_INVALID_ARGUMENT, "null pointer");
+  LaunchSlots s;
+  for (uint32_t i = 0; i < n; ++i) out[i] = s.take(captured[i] != 0);
   return DTO_OK;
 }
 

@@ -118,7 +118,7 @@ static hipError_t launch_t(dto_job *j, uint32_t grid, hipStream_t st, const uint
   auto kern = k_cut<NT, E, BUILD>;
   const LdsLayout &lo = j->lo_cut;
   (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lo.total);
-  uint32_t *ctr = j->d_ctr + (j->ctr_next.fetch_add(1u) % kCounterRing);
+  uint32_t *ctr = j->d_ctr + j->slots.take(st);
   StagingOrder order(j, lo, st);
   hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, ctr);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lo.total, st, j->dev, lo, i1, i2, n_perm, base, seed, job_id, permuted,

@@ -46,7 +46,24 @@ int cut_shape(const HostJob *const *jobs, size_t n, size_t lds_limit, CutShape *
 void cut_levels(const HostJob &h, DevJob &d);
 }  // namespace dto
 
-constexpr uint32_t kCounterRing = 256;
+/* Slots of a job's work counters (and of its partial results), one per
+ * launch, so that launches on different streams do not share one: a ring for
+ * launches that run at once, and one for captured launches, which keep their
+ * slot for every replay and would otherwise share it with each 256th ordinary
+ * launch.  Only more launches in flight at once than the ring has slots, or
+ * replays of captured launches more than kCaptureRing apart, meet. */
+constexpr uint32_t kCounterRing = 256, kCaptureRing = 64, kCounterSlots = kCounterRing + kCaptureRing;
+struct LaunchSlots {
+  std::atomic<uint32_t> ordinary{0}, captured{0};
+  uint32_t take(bool capturing) {
+    return capturing ? kCounterRing + captured.fetch_add(1u) % kCaptureRing : ordinary.fetch_add(1u) % kCounterRing;
+  }
+  uint32_t take(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+    return take(cs != hipStreamCaptureStatusNone);
+  }
+};
 /* A resident job's room for small calls (upload_job): bytes of the error
  * word's block, and records after it (a run of 1,000 permutations). */
 constexpr size_t kErrBytes = 256, kCallRecords = 1025;
@@ -76,11 +93,8 @@ struct dto_job {
   std::vector<unsigned char> image; /* the arena's contents (kept for deferred jobs) */
   ArenaOffsets off{};
   int *d_err = nullptr;
-  /* work counters of permutation launches: a ring of kCounterRing slots, one
-   * per launch, so that launches on different streams do not share one (a
-   * job with more launches than that in flight at once would) */
-  uint32_t *d_ctr = nullptr;
-  std::atomic<uint32_t> ctr_next{0};
+  uint32_t *d_ctr = nullptr; /* work counters of permutation launches, kCounterSlots */
+  LaunchSlots slots;
   int device = -1;
   dto::LdsLayout lo_screen{}, lo_plain{}; /* lo_screen: a server's slices */
   dto::CutShape cut_sh{};

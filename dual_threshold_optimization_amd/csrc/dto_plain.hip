@@ -13,16 +13,15 @@
 using namespace dto;
 
 /* Launches of at most kSplitTasks tasks split each over several workgroups,
- * kSplitItems in all (two for each CU); their partial results go to one of
- * kCounterRing slots of a buffer that the job keeps from its first plain
- * launch on. */
+ * kSplitItems in all (two for each CU); their partial results go to the
+ * launch's slot of a buffer that the job keeps from its first plain launch on. */
 constexpr uint32_t kSplitTasks = 256, kSplitItems = 512;
 
 /* The launch's slot of the partial buffer, or NULL where there is no memory
  * for it (the launch is then not split). */
 static BestKey *partial_slot(dto_job *j, uint32_t slot) {
   std::lock_guard<std::mutex> g(j->cut_mu);
-  if (!j->partial && j->alloc(&j->partial, (size_t)kCounterRing * kSplitItems * sizeof(BestKey)) != hipSuccess) {
+  if (!j->partial && j->alloc(&j->partial, (size_t)kCounterSlots * kSplitItems * sizeof(BestKey)) != hipSuccess) {
     (void)hipGetLastError();
     j->partial = nullptr;
     return nullptr;
@@ -37,7 +36,7 @@ static hipError_t launch_t(dto_job *j, uint32_t max_grid, hipStream_t st, const 
   auto kern = k_plain<kNT, E, PL>;
   const LdsLayout &lo = j->lo_plain;
   (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lo.total);
-  const uint32_t slot = j->ctr_next.fetch_add(1u) % kCounterRing;
+  const uint32_t slot = j->slots.take(st);
   uint32_t *ctr = j->d_ctr + slot;
   uint32_t parts = 1;
   BestKey *partial = nullptr;

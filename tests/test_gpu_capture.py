@@ -48,3 +48,32 @@ def test_first_launch_during_a_global_capture(dto, gpu, mode, inside):
         torch.cuda.synchronize()
     job.close()
     ref.close()
+
+
+@pytest.mark.parametrize("mode", ["screened", "plain"])
+def test_replay_among_many_ordinary_launches(dto, gpu, mode):
+    """A captured launch replayed while ordinary launches of the same job, more
+    than the ring of counters has slots, run on another stream."""
+    import torch
+    P, n = 100, 2000
+    job = _job(dto, n)
+    want, got = _records(torch, P), _records(torch, P)
+    one_want, one = _records(torch, 1), _records(torch, 300)
+    job.run_device(P, want.data_ptr(), seed=3, mode=mode)
+    job.run_device(1, one_want.data_ptr(), seed=9, mode=mode)
+    other, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        job.run_device(P, got.data_ptr(), seed=3, mode=mode, stream=torch.cuda.current_stream().cuda_stream)
+    for _ in range(2):
+        got.zero_()
+        one.zero_()
+        torch.cuda.synchronize()
+        for q in range(300):
+            if q % 30 == 0:
+                graph.replay()
+            job.run_device(1, one.data_ptr() + q * REC, seed=9, mode=mode, stream=other.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert torch.equal(one.view(300, REC), one_want.expand(300, REC))
+    job.close()
