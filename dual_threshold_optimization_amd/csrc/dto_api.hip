@@ -150,6 +150,7 @@ int prepare_job(dto_job *j) {
   (void)cut_layout(h, j->cut_sh.nt / 64, j->cut_sh.build, &j->lo_cut);
   if (j->cut) (void)hipFree(j->cut);
   j->cut = nullptr;
+  j->cut_pending = false;
   std::vector<unsigned char> &buf = j->image;
   buf.clear();
   ArenaOffsets &o = j->off;
@@ -239,7 +240,7 @@ int upload_job(dto_job *j) {
   bind_job(j, (unsigned char *)j->arena);
   j->d_err = (int *)((unsigned char *)j->arena + tables);
   std::vector<unsigned char>().swap(j->image); /* the device copy is the job's now */
-  return ensure_cut(j, 0);
+  return DTO_OK;
 }
 
 int ensure_resident(dto_job *j) {
@@ -275,10 +276,16 @@ static int launch_perms(dto_job *j, uint32_t mode, bool expl, const uint32_t *d1
     const uint32_t g = perm_grid(j, j->lo_plain, ~0ull, 4);
     e = launch_plain(j, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
   } else if (mode == DTO_MODE_SCREENED) {
-    int rc = ensure_cut(j, st);
+    const uint32_t *cut = nullptr;
+    int rc = cut_tables(j, st, &cut);
     if (rc) return rc;
+    if (!cut) {
+      /* no memory for the tables: the plain kernels give the same records */
+      if (lead && (rc = launch_perms(j, DTO_MODE_PLAIN, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_out, st))) return rc;
+      return launch_perms(j, DTO_MODE_PLAIN, expl, d1, d2, n_perm, base, seed, job_id, permuted, d_out + lead, st);
+    }
     const uint32_t g = perm_grid(j, j->lo_cut, n_perm + lead, j->cut_sh.nt == 512 ? 4 : 2);
-    e = launch_cut(j, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, lead, d_out);
+    e = launch_cut(j, cut, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, lead, d_out);
   } else {
     return fail(DTO_ERR_INVALID_ARGUMENT, "unknown mode");
   }
@@ -635,6 +642,7 @@ void dto_job_destroy(dto_job *job) {
   if (job->cut) (void)hipFree(job->cut);
   if (job->partial) (void)hipFree(job->partial);
   if (job->ws_ev) (void)hipEventDestroy(job->ws_ev);
+  if (job->cut_ev) (void)hipEventDestroy(job->cut_ev);
   delete job;
 }
 

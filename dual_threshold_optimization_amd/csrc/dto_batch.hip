@@ -37,8 +37,6 @@ using namespace dto;
 
 namespace {
 
-/* Launch shapes of a server's slices: the screen table in LDS or not, the
- * bins and the pair staging in LDS or global memory. */
 /* Global buffers of a launch: pair staging (ws, ws_stride u16 per
  * workgroup) and bins arrays (gnb, gnb_stride u16 per workgroup). */
 struct Globals {
@@ -57,9 +55,12 @@ hipError_t launch_slice_t(uint32_t grid, uint32_t lds, hipStream_t st, const Bat
   return hipGetLastError();
 }
 
+/* The first-term kernels' launch shapes: the screen table in LDS or not (hl),
+ * the bins (nbl) and the pair staging (pl) in LDS or global memory, every
+ * job's lane segment in registers or not (rc). */
 hipError_t launch_slice(bool hl, bool nbl, bool pl, bool rc, uint32_t grid, uint32_t lds, hipStream_t st,
-                          const BatchJob *jobs, const WorkItem *items, uint32_t n_items, uint64_t seed,
-                          uint32_t *counter, int *err, const Globals &g) {
+                        const BatchJob *jobs, const WorkItem *items, uint32_t n_items, uint64_t seed,
+                        uint32_t *counter, int *err, const Globals &g) {
   if (hl && nbl)
     return rc ? launch_slice_t<kNT, true, true, true, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g)
               : launch_slice_t<kNT, true, true, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
@@ -73,25 +74,56 @@ hipError_t launch_slice(bool hl, bool nbl, bool pl, bool rc, uint32_t grid, uint
             : launch_slice_t<kNT, false, false, false, true>(grid, lds, st, jobs, items, n_items, seed, counter, err, g);
 }
 
-/* One launch shape for all jobs of a batch, with each job's layout. */
+/* One launch shape for all jobs of a batch, with each job's layout: of the
+ * cut kernels, or, where a job's cut tables found no memory, of the
+ * first-term kernels. */
 struct Shape {
-  CutShape cut;
-  uint32_t max_n2 = 0; /* largest N2 */
+  bool cut = true;
+  CutShape sh;                               /* cut kernels; nt and lds hold for both */
+  bool hl = true, nbl = true, pl = true, rc = true; /* first-term kernels */
+  uint32_t max_n2 = 0, max_n = 0;            /* largest N2, largest max(N1, N2) */
   std::vector<LdsLayout> lo;
 };
 
 int plan_shape(const std::vector<dto_job *> &jobs, size_t lds_limit, Shape &s) {
-  std::vector<const HostJob *> hs;
-  for (dto_job *j : jobs) hs.push_back(&j->h);
-  int rc = cut_shape(hs.data(), hs.size(), lds_limit, &s.cut);
-  if (rc) return rc;
-  s.max_n2 = 1;
+  s.max_n2 = s.max_n = 1;
   s.lo.clear();
   for (dto_job *j : jobs) {
-    LdsLayout L;
-    (void)cut_layout(j->h, s.cut.nt / 64, s.cut.build, &L);
-    s.lo.push_back(L);
     s.max_n2 = std::max(s.max_n2, j->dev.N2);
+    s.max_n = std::max(s.max_n, std::max(j->dev.N1, j->dev.N2));
+  }
+  if (s.cut) {
+    std::vector<const HostJob *> hs;
+    for (dto_job *j : jobs) hs.push_back(&j->h);
+    int rc = cut_shape(hs.data(), hs.size(), lds_limit, &s.sh);
+    if (rc) return rc;
+    for (dto_job *j : jobs) {
+      LdsLayout L;
+      (void)cut_layout(j->h, s.sh.nt / 64, s.sh.build, &L);
+      s.lo.push_back(L);
+    }
+    s.pl = s.lo.empty() || s.lo[0].pairs_in_lds;
+    s.nbl = true;
+    return DTO_OK;
+  }
+  /* the first of (table and bins in LDS), (table in LDS, bins global), (table
+   * global) that every job fits */
+  bool fit_hb = true, fit_h = true;
+  s.rc = s.pl = true;
+  for (dto_job *j : jobs) {
+    if ((j->dev.T2w + 63) / 64 > kSegWords) s.rc = false;
+    if (make_layout(j->h, kNT / 64, true, lds_limit, true).total > lds_limit) fit_hb = false;
+    if (make_layout(j->h, kNT / 64, true, lds_limit, false).total > lds_limit) fit_h = false;
+  }
+  s.hl = fit_h;
+  s.nbl = fit_hb || !fit_h;
+  s.sh = {kNT, 0, 0};
+  for (dto_job *j : jobs) {
+    const LdsLayout L = make_layout(j->h, kNT / 64, s.hl, lds_limit, s.nbl);
+    if (L.total > lds_limit) return fail(DTO_ERR_TOO_LARGE, "job does not fit in LDS");
+    if (!L.pairs_in_lds) s.pl = false;
+    s.lo.push_back(L);
+    s.sh.lds = std::max(s.sh.lds, L.total);
   }
   return DTO_OK;
 }
@@ -131,7 +163,8 @@ struct dto_batch {
   uint32_t *d_counter = nullptr;
   int *d_err = nullptr;
   dto_record *d_out = nullptr;
-  uint16_t *d_ws = nullptr; /* global pair staging when the LDS cannot hold the pairs */
+  uint16_t *d_ws = nullptr;  /* global pair staging when the LDS cannot hold the pairs */
+  uint16_t *d_gnb = nullptr; /* global bins arrays when it holds the screen table but not the bins */
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
   hipStream_t own_stream = nullptr;
@@ -145,9 +178,11 @@ static void batch_free_plan(dto_batch *b) {
   if (b->d_jobs) (void)hipFree(b->d_jobs);
   if (b->d_items) (void)hipFree(b->d_items);
   if (b->d_ws) (void)hipFree(b->d_ws);
+  if (b->d_gnb) (void)hipFree(b->d_gnb);
   b->d_jobs = nullptr;
   b->d_items = nullptr;
   b->d_ws = nullptr;
+  b->d_gnb = nullptr;
 }
 
 /* Queue reset, then the persistent kernel. */
@@ -155,8 +190,13 @@ static hipError_t batch_kernels(const dto_batch *b, hipStream_t st) {
   hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, st, b->d_counter, b->d_err);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return launch_batch_cut(b->shape.cut, b->grid, st, b->d_jobs, b->d_items, b->n_items, b->seed, b->d_counter,
-                          b->d_err, b->d_ws, b->shape.max_n2);
+  const Shape &s = b->shape;
+  if (s.cut)
+    return launch_batch_cut(s.sh, b->grid, st, b->d_jobs, b->d_items, b->n_items, b->seed, b->d_counter, b->d_err,
+                            b->d_ws, s.max_n2);
+  const Globals g = {b->d_ws, b->d_gnb, s.max_n2, s.max_n};
+  return launch_slice(s.hl, s.nbl, s.pl, s.rc, b->grid, s.sh.lds, st, b->d_jobs, b->d_items, b->n_items, b->seed,
+                      b->d_counter, b->d_err, g);
 }
 
 /* Builds the job table and the work queue for the current shape and chunk. */
@@ -167,6 +207,7 @@ static int batch_plan(dto_batch *b) {
   std::vector<BatchJob> hj(b->jobs.size());
   for (size_t i = 0; i < b->jobs.size(); ++i) {
     hj[i].J = b->jobs[i]->dev;
+    hj[i].J.cut = b->shape.cut ? b->jobs[i]->cut : nullptr;
     hj[i].lo = b->shape.lo[i];
     hj[i].out = b->d_out + b->out_off[i];
     hj[i].n_perm = (uint32_t)b->n_perm[i];
@@ -196,8 +237,9 @@ static int batch_plan(dto_batch *b) {
   HIP_TRY(hipMalloc(&b->d_items, std::max<size_t>(1, items.size()) * sizeof(WorkItem)));
   HIP_TRY(hipMemcpy(b->d_jobs, hj.data(), hj.size() * sizeof(BatchJob), hipMemcpyHostToDevice));
   if (!items.empty()) HIP_TRY(hipMemcpy(b->d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
-  b->grid = grid_for(b->cus, b->shape.cut.lds, b->shape.cut.nt, b->n_items);
-  if (!b->shape.lo.empty() && !b->shape.lo[0].pairs_in_lds) HIP_TRY(hipMalloc(&b->d_ws, (size_t)b->grid * b->shape.max_n2 * sizeof(uint16_t)));
+  b->grid = grid_for(b->cus, b->shape.sh.lds, b->shape.sh.nt, b->n_items);
+  if (!b->shape.pl) HIP_TRY(hipMalloc(&b->d_ws, (size_t)b->grid * b->shape.max_n2 * sizeof(uint16_t)));
+  if (!b->shape.nbl) HIP_TRY(hipMalloc(&b->d_gnb, (size_t)b->grid * b->shape.max_n * sizeof(uint16_t)));
   return DTO_OK;
 }
 
@@ -222,10 +264,12 @@ int dto_batch_create(dto_job *const *jobs, const uint64_t *n_perm, uint64_t n_jo
       delete b;
       return fail(DTO_ERR_INVALID_ARGUMENT, "bad job or permutation count");
     }
-    if ((rc = ensure_resident(jobs[i])) || (rc = ensure_cut(jobs[i], 0))) {
+    const uint32_t *cut = nullptr;
+    if ((rc = ensure_resident(jobs[i])) || (rc = cut_tables(jobs[i], 0, &cut))) {
       delete b;
       return rc;
     }
+    if (!cut) b->shape.cut = false;
     b->jobs.push_back(jobs[i]);
     b->n_perm.push_back(n_perm[i]);
     b->out_off.push_back(b->total_tasks);
@@ -236,7 +280,10 @@ int dto_batch_create(dto_job *const *jobs, const uint64_t *n_perm, uint64_t n_jo
     dto_batch_destroy(b);
     return fail(DTO_ERR_DEVICE, "hipMalloc failed for batch buffers");
   }
-  if ((rc = batch_plan(b))) {
+  rc = batch_plan(b);
+  /* the tables are complete before a launch on any stream reads them */
+  if (!rc && hipStreamSynchronize(0) != hipSuccess) rc = fail(DTO_ERR_DEVICE, "cut tables of a batch");
+  if (rc) {
     dto_batch_destroy(b);
     return rc;
   }
@@ -317,7 +364,7 @@ int dto_batch_autotune(dto_batch *b, int *waves) {
   (void)hipEventDestroy(e1);
   b->chunk = best_chunk;
   int rc = batch_plan(b);
-  if (waves) *waves = b->shape.cut.nt / 64;
+  if (waves) *waves = b->shape.sh.nt / 64;
   return rc;
 }
 

@@ -4,7 +4,7 @@
  *
  * For one job every cell (i, j) has fixed K_i, n_j and N, so whether its tail
  * P(X >= k) can lie at or below a level e^L depends on k alone.  The job's cut
- * tables (k_cut_table, built once when its tables are uploaded) hold, for each
+ * tables (k_cut_table, built once by its first screened launch) hold, for each
  * of a few levels, the largest k whose tail is certain to lie above the level;
  * level 0 drops only cells whose tail is exactly 1.  A permutation is swept
  * against the start level's table: per pair of columns the screen is one

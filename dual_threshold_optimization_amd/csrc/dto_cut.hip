@@ -90,49 +90,77 @@ void dto::cut_levels(const HostJob &h, DevJob &d) {
   for (uint32_t l = 0; l < kCutLevels; ++l) d.cut_level[l] = (float)level[l];
 }
 
-int dto::ensure_cut(dto_job *j, hipStream_t st) {
+int dto::cut_tables(dto_job *j, hipStream_t st, const uint32_t **out) {
   std::lock_guard<std::mutex> g(j->cut_mu);
-  if (j->cut) return DTO_OK;
+  *out = j->cut;
+  if (j->cut && !j->cut_pending) return DTO_OK;
+  RelaxedCapture relaxed;
+  const bool capturing = stream_capturing(st);
+  if (j->cut) {
+    const hipError_t q = hipEventQuery(j->cut_ev);
+    if (q == hipSuccess) {
+      j->cut_pending = false;
+      return DTO_OK;
+    }
+    (void)hipGetLastError();
+    if (q != hipErrorNotReady) return fail(DTO_ERR_DEVICE, std::string("cut tables: ") + hipGetErrorString(q));
+    /* a capture cannot wait on work recorded outside it */
+    if (capturing) HIP_TRY(hipEventSynchronize(j->cut_ev));
+    else HIP_TRY(hipStreamWaitEvent(st, j->cut_ev, 0));
+    return DTO_OK;
+  }
   const size_t per_level = (size_t)j->dev.T1 * j->dev.cut_segs * 2u * kCutSpan;
+  if (!j->cut_ev) HIP_TRY(hipEventCreateWithFlags(&j->cut_ev, hipEventDisableTiming));
   void *p = nullptr;
   /* the sweep loads one row's segment past the last */
-  HIP_TRY(j->alloc(&p, (kCutLevels * per_level + 2u * kCutSpan) * sizeof(uint16_t)));
-  const uint32_t grid = (uint32_t)std::min<size_t>((per_level + 255) / 256, 65536);
-  hipLaunchKernelGGL(k_cut_table, dim3(grid), dim3(256), 0, st, j->dev, (uint16_t *)p);
-  hipError_t e = hipGetLastError();
-  /* complete before any launch on any stream reads it */
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (j->alloc(&p, (kCutLevels * per_level + 2u * kCutSpan) * sizeof(uint16_t)) != hipSuccess) {
+    (void)hipGetLastError();
+    return DTO_OK;
+  }
+  /* a captured launch would only build them when it is replayed: they are
+   * built beside the capture, and are complete before it goes on */
+  hipStream_t b = st;
+  hipError_t e = capturing ? hipStreamCreateWithFlags(&b, hipStreamNonBlocking) : hipSuccess;
+  if (e == hipSuccess) {
+    const uint32_t grid = (uint32_t)std::min<size_t>((per_level + 255) / 256, 65536);
+    hipLaunchKernelGGL(k_cut_table, dim3(grid), dim3(256), 0, b, j->dev, (uint16_t *)p);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = capturing ? hipStreamSynchronize(b) : hipEventRecord(j->cut_ev, b);
+    if (capturing) (void)hipStreamDestroy(b);
+  }
   if (e != hipSuccess) {
     (void)hipFree(p);
     return fail(DTO_ERR_DEVICE, std::string("cut tables: ") + hipGetErrorString(e));
   }
-  j->dev.cut = (const uint32_t *)p;
-  j->cut = p;
+  *out = j->cut = (uint32_t *)p;
+  j->cut_pending = !capturing;
   return DTO_OK;
 }
 
 template <int NT, int BUILD, bool E>
-static hipError_t launch_t(dto_job *j, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
+static hipError_t launch_t(dto_job *j, const uint32_t *cut, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
                            uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted,
                            uint32_t lead, dto_record *out) {
   auto kern = k_cut<NT, E, BUILD>;
   const LdsLayout &lo = j->lo_cut;
   (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lo.total);
   uint32_t *ctr = j->d_ctr + j->slots.take(st);
+  DevJob dev = j->dev;
+  dev.cut = cut;
   StagingOrder order(j, lo, st);
   hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, ctr);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lo.total, st, j->dev, lo, i1, i2, n_perm, base, seed, job_id, permuted,
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lo.total, st, dev, lo, i1, i2, n_perm, base, seed, job_id, permuted,
                      lead, out, j->d_err, j->ws, ctr);
   return hipGetLastError();
 }
 
-hipError_t dto::launch_cut(dto_job *j, bool expl, uint32_t grid, hipStream_t st, const uint32_t *i1,
-                           const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id,
+hipError_t dto::launch_cut(dto_job *j, const uint32_t *cut, bool expl, uint32_t grid, hipStream_t st,
+                           const uint32_t *i1, const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id,
                            int32_t permuted, uint32_t lead, dto_record *out) {
 #define DTO_CUT(NT, B)                                                                                               \
   if (j->cut_sh.nt == NT && j->cut_sh.build == B)                                                                    \
-    return expl ? launch_t<NT, B, true>(j, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, lead, out)        \
-                : launch_t<NT, B, false>(j, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, lead, out);
+    return expl ? launch_t<NT, B, true>(j, cut, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, lead, out)   \
+                : launch_t<NT, B, false>(j, cut, grid, st, i1, i2, n_perm, base, seed, job_id, permuted, lead, out);
   DTO_CUT(512, kBuildRegs)
   DTO_CUT(512, kBuildLds)
   DTO_CUT(512, kBuildGlobal)

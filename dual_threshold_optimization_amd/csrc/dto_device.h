@@ -41,7 +41,7 @@ struct DevJob {
   const float *H32;         /* [N+1] LF[x] - x*(ln N - 1), rounded to f32 */
   const float *A32;         /* [T1] H(K_i) + H(N-K_i) */
   const float *B32;         /* [T2] H(n_j) + H(N-n_j) - H(N) */
-  const uint32_t *cut;      /* the cut tables of the screened kernels (dto_cut.h) */
+  const uint32_t *cut;      /* the cut tables of the screened kernels (dto_cut.h), set for a launch */
   uint32_t cut_segs;        /* column segments per row in them */
   float cut_level[kCutLevels]; /* log p level of each, falling; 0: p == 1 cells only */
   unsigned long long *stats; /* [16] work counters (dto_internal_stats) */

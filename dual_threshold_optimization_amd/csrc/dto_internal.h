@@ -46,6 +46,12 @@ int cut_shape(const HostJob *const *jobs, size_t n, size_t lds_limit, CutShape *
 void cut_levels(const HostJob &h, DevJob &d);
 }  // namespace dto
 
+inline bool stream_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+  return cs != hipStreamCaptureStatusNone;
+}
+
 /* Slots of a job's work counters (and of its partial results), one per
  * launch, so that launches on different streams do not share one: a ring for
  * launches that run at once, and one for captured launches, which keep their
@@ -58,11 +64,7 @@ struct LaunchSlots {
   uint32_t take(bool capturing) {
     return capturing ? kCounterRing + captured.fetch_add(1u) % kCaptureRing : ordinary.fetch_add(1u) % kCounterRing;
   }
-  uint32_t take(hipStream_t st) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
-    return take(cs != hipStreamCaptureStatusNone);
-  }
+  uint32_t take(hipStream_t st) { return take(stream_capturing(st)); }
 };
 /* A resident job's room for small calls (upload_job): bytes of the error
  * word's block, and records after it (a run of 1,000 permutations). */
@@ -99,7 +101,11 @@ struct dto_job {
   dto::LdsLayout lo_screen{}, lo_plain{}; /* lo_screen: a server's slices */
   dto::CutShape cut_sh{};
   dto::LdsLayout lo_cut{};
-  void *cut = nullptr; /* the cut tables (dev.cut), set under cut_mu */
+  /* the cut tables, set under cut_mu by the first screened launch; while
+   * cut_pending, launches on other streams wait for cut_ev first */
+  uint32_t *cut = nullptr;
+  hipEvent_t cut_ev = nullptr;
+  bool cut_pending = false;
   void *partial = nullptr; /* split plain launches' partial results, set under cut_mu */
   std::mutex cut_mu;
   uint16_t *ws = nullptr; /* global pair staging (only when the LDS cannot hold the pairs) */
@@ -139,10 +145,7 @@ struct StagingOrder {
   hipStream_t st;
   bool on = false;
   StagingOrder(const dto_job *job, const dto::LdsLayout &lo, hipStream_t s) : j(const_cast<dto_job *>(job)), st(s) {
-    if (lo.pairs_in_lds || !j->ws_ev) return;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
-    if (cs != hipStreamCaptureStatusNone) return;
+    if (lo.pairs_in_lds || !j->ws_ev || stream_capturing(st)) return;
     j->ws_mu.lock();
     on = true;
     if (j->ws_used) (void)hipStreamWaitEvent(st, j->ws_ev, 0);
@@ -160,10 +163,11 @@ namespace dto {
  * record into out; an out-of-range permutation index sets *err. */
 hipError_t launch_grid(dto_job *job, const uint32_t *d1, const uint32_t *d2, uint32_t *kcnt, dto_record *out, int *err,
                        hipStream_t st);
-/* Builds a job's cut tables on a stream if it has none yet; they are complete
- * on return. */
-int ensure_cut(dto_job *j, hipStream_t st);
-hipError_t launch_cut(dto_job *j, bool expl, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
+/* A job's cut tables for work on stream st: built there if it has none yet,
+ * and st waits where another stream still builds them.  *out is NULL where
+ * the device has no memory for them. */
+int cut_tables(dto_job *j, hipStream_t st, const uint32_t **out);
+hipError_t launch_cut(dto_job *j, const uint32_t *cut, bool expl, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
                       uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted, uint32_t lead,
                       dto_record *out);
 hipError_t launch_plain(dto_job *j, bool expl, uint32_t max_grid, hipStream_t st, const uint32_t *i1,

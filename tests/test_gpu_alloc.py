@@ -30,3 +30,87 @@ def test_upload_fails_then_succeeds(dto, gpu, nth):
     assert job.optimize(mode="plain") == want.optimize(mode="plain")
     job.close()
     want.close()
+
+
+def _same(a, b):
+    return bytes(a[0]) == bytes(b[0]) and a[1].tobytes() == b[1].tobytes()
+
+
+@pytest.mark.parametrize("n", [50, 3000, 24000])
+def test_no_memory_for_cut_tables(dto, gpu, n):
+    """Screened calls of a job whose cut tables found no memory: the same
+    records, and tables again once there is memory."""
+    want = dto.Job.from_lists(*_lists(n))
+    P = 4
+    rng = np.random.default_rng(n)
+    idx = dict(idx1=np.stack([rng.permutation(n) for _ in range(P)]), idx2=np.stack([rng.permutation(n) for _ in range(P)]))
+    for call in (lambda j: j.run(P, seed=7), lambda j: j.run(P, **idx)):
+        job = dto.Job.from_lists(*_lists(n))
+        _fail_alloc(dto, job, 1)
+        assert _same(call(job), call(want))
+        assert _same(call(job), call(want))
+        job.close()
+    job = dto.Job.from_lists(*_lists(n))
+    _fail_alloc(dto, job, 1)
+    assert job.optimize() == want.optimize()
+    job.close()
+    want.close()
+
+
+# the first-term kernels' shapes: table and bins in LDS, table in LDS, table
+# global with the pairs in LDS, all global
+@pytest.mark.parametrize("n", [1500, 22000, 27000, 36000])
+def test_batch_without_cut_tables(dto, gpu, n):
+    """A batch with one job whose cut tables found no memory."""
+    sizes, perms = [300, n, 40], [5, 3, 9]
+    res = []
+    for nth in (0, 1):
+        jobs = [dto.Job.from_lists(*_lists(m)) for m in sizes]
+        _fail_alloc(dto, jobs[1], nth)
+        b = dto.Batch(jobs, perms, seed=6)
+        for rep in range(2):
+            b.launch()
+            res.append([bytes(r) for r in b.results()])
+            if nth:
+                b.autotune()
+        b.close()
+        for j in jobs:
+            j.close()
+    assert all(r == res[0] for r in res)
+
+
+@pytest.mark.parametrize("nth", [2, 3])
+def test_creation_needs_no_cut_tables(dto, gpu, nth):
+    """An upload at this size makes one allocation.  The next are the split
+    plain launches' partial results and, from the first screened call on, the
+    cut tables: calls that can do without them do."""
+    job = dto.Job.from_lists(*_lists(3000), defer_upload=True)
+    _fail_alloc(dto, job, nth)
+    want = dto.Job.from_lists(*_lists(3000))
+    assert job.optimize(mode="plain") == want.optimize(mode="plain")
+    assert job.process_threshold_pairs().tobytes() == want.process_threshold_pairs().tobytes()
+    assert job.optimize() == want.optimize()
+    job.close()
+    want.close()
+
+
+@pytest.mark.parametrize("n", [900, 20000])
+def test_first_launches_on_two_streams(dto, gpu, n):
+    """The first screened launch builds the tables on its stream; one right
+    after it on another stream waits for them."""
+    import torch
+    P = 6
+    want = dto.Job.from_lists(*_lists(n))
+    w = torch.zeros(P * 72, dtype=torch.uint8, device="cuda:0")
+    want.run_device(P, w.data_ptr(), seed=3)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        job = dto.Job.from_lists(*_lists(n))
+        outs, streams = [torch.zeros_like(w) for _ in range(3)], [torch.cuda.Stream() for _ in range(3)]
+        torch.cuda.synchronize()
+        for o, st in zip(outs, streams):
+            job.run_device(P, o.data_ptr(), seed=3, stream=st.cuda_stream)
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, w) for o in outs)
+        job.close()
+    want.close()
