@@ -150,6 +150,7 @@ int prepare_job(dto_job *j) {
   (void)cut_layout(h, j->cut_sh.nt / 64, j->cut_sh.build, &j->lo_cut);
   if (j->cut) (void)hipFree(j->cut);
   j->cut = nullptr;
+  j->cut_bytes = 0;
   j->cut_pending = false;
   std::vector<unsigned char> &buf = j->image;
   buf.clear();
@@ -221,12 +222,15 @@ int upload_job(dto_job *j) {
   if (j->ws) (void)hipFree(j->ws);
   j->arena = nullptr;
   j->ws = nullptr;
+  j->own_bytes = j->ws_bytes = 0;
   j->resident = false;
   /* global pair staging for layouts whose pairs do not fit in LDS; before the
    * job is resident, so that no launch finds it missing */
   j->ws_slots = (uint32_t)pr.cus * 4u;
   if (!j->lo_plain.pairs_in_lds || !j->lo_cut.pairs_in_lds) {
-    HIP_TRY(j->alloc((void **)&j->ws, (size_t)j->ws_slots * std::max<uint32_t>(j->dev.N2, 1) * sizeof(uint16_t)));
+    const size_t ws_bytes = (size_t)j->ws_slots * std::max<uint32_t>(j->dev.N2, 1) * sizeof(uint16_t);
+    HIP_TRY(j->alloc((void **)&j->ws, ws_bytes));
+    j->ws_bytes = ws_bytes;
     if (!j->ws_ev) HIP_TRY(hipEventCreateWithFlags(&j->ws_ev, hipEventDisableTiming));
   }
   /* after the tables: the error word, the records of a small run and one
@@ -234,8 +238,10 @@ int upload_job(dto_job *j) {
    * one copy brings the error word and the records back */
   const size_t tables = j->image.size();
   j->image.resize(tables + kErrBytes, 0);
-  HIP_TRY(j->alloc(&j->arena, j->image.size() + kCallRecords * sizeof(dto_record) +
-                                  ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t)));
+  const size_t own_bytes = j->image.size() + kCallRecords * sizeof(dto_record) +
+                           ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t);
+  HIP_TRY(j->alloc(&j->arena, own_bytes));
+  j->own_bytes = own_bytes;
   HIP_TRY(hipMemcpy(j->arena, j->image.data(), j->image.size(), hipMemcpyHostToDevice));
   bind_job(j, (unsigned char *)j->arena);
   j->d_err = (int *)((unsigned char *)j->arena + tables);
@@ -623,7 +629,10 @@ int dto_job_info_get(const dto_job *job, dto_job_info *info) {
   info->n_thresholds2 = (uint32_t)job->h.thr2.size();
   info->dropped1 = job->h.dropped1;
   info->dropped2 = job->h.dropped2;
-  info->device_bytes = job->arena_bytes;
+  std::lock_guard<std::mutex> g(const_cast<dto_job *>(job)->cut_mu);
+  /* a job without an arena of its own: what it takes of a server's pool */
+  info->device_bytes = (job->own_bytes ? job->own_bytes : job->arena_bytes) + job->ws_bytes + job->cut_bytes +
+                       job->partial_bytes;
   return DTO_OK;
 }
 

@@ -113,7 +113,8 @@ int dto::cut_tables(dto_job *j, hipStream_t st, const uint32_t **out) {
   if (!j->cut_ev) HIP_TRY(hipEventCreateWithFlags(&j->cut_ev, hipEventDisableTiming));
   void *p = nullptr;
   /* the sweep loads one row's segment past the last */
-  if (j->alloc(&p, (kCutLevels * per_level + 2u * kCutSpan) * sizeof(uint16_t)) != hipSuccess) {
+  const size_t bytes = (kCutLevels * per_level + 2u * kCutSpan) * sizeof(uint16_t);
+  if (j->alloc(&p, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return DTO_OK;
   }
@@ -133,6 +134,7 @@ int dto::cut_tables(dto_job *j, hipStream_t st, const uint32_t **out) {
     return fail(DTO_ERR_DEVICE, std::string("cut tables: ") + hipGetErrorString(e));
   }
   *out = j->cut = (uint32_t *)p;
+  j->cut_bytes = bytes;
   j->cut_pending = !capturing;
   return DTO_OK;
 }

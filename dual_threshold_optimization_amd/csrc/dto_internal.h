@@ -91,6 +91,9 @@ struct dto_job {
   dto::DevJob dev{};
   void *arena = nullptr;
   size_t arena_bytes = 0; /* size of the arena image */
+  /* sizes of the job's own allocations, 0 where there is none; those of the
+   * cut tables and partial results under cut_mu */
+  size_t own_bytes = 0, ws_bytes = 0, cut_bytes = 0, partial_bytes = 0;
   bool resident = false;  /* dev points at an arena (own or pooled) */
   std::vector<unsigned char> image; /* the arena's contents (kept for deferred jobs) */
   ArenaOffsets off{};

@@ -21,10 +21,14 @@ constexpr uint32_t kSplitTasks = 256, kSplitItems = 512;
  * for it (the launch is then not split). */
 static BestKey *partial_slot(dto_job *j, uint32_t slot) {
   std::lock_guard<std::mutex> g(j->cut_mu);
-  if (!j->partial && j->alloc(&j->partial, (size_t)kCounterSlots * kSplitItems * sizeof(BestKey)) != hipSuccess) {
-    (void)hipGetLastError();
-    j->partial = nullptr;
-    return nullptr;
+  if (!j->partial) {
+    const size_t bytes = (size_t)kCounterSlots * kSplitItems * sizeof(BestKey);
+    if (j->alloc(&j->partial, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      j->partial = nullptr;
+      return nullptr;
+    }
+    j->partial_bytes = bytes;
   }
   return (BestKey *)j->partial + (size_t)slot * kSplitItems;
 }

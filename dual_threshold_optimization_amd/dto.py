@@ -61,7 +61,16 @@ class Job:
         self.len1, self.len2 = info.len1, info.len2
         self.n_thresholds1, self.n_thresholds2 = info.n_thresholds1, info.n_thresholds2
         self.dropped1, self.dropped2 = info.dropped1, info.dropped2
-        self.device_bytes = info.device_bytes
+        self._device_bytes = info.device_bytes
+
+    @property
+    def device_bytes(self):
+        """The job's device footprint at this time; after close() or release(), the last one read."""
+        if self._h is not None:
+            info = _lib.JobInfo()
+            _lib.check(_lib.lib().dto_job_info_get(self._h, ctypes.byref(info)))
+            self._device_bytes = info.device_bytes
+        return self._device_bytes
 
     # ---- construction -------------------------------------------------------
     @classmethod

@@ -89,7 +89,9 @@ typedef struct {
   uint64_t len1, len2;      /* list lengths after any background drop */
   uint32_t n_thresholds1, n_thresholds2;
   uint64_t dropped1, dropped2; /* features dropped (DTO_DROP_OUTSIDE_BACKGROUND) */
-  uint64_t device_bytes;       /* resident device footprint of the job */
+  uint64_t device_bytes;       /* device footprint of the job: its tables and call room (before its
+                                  upload, or in a server: its tables), and what launches so far have
+                                  added (screened: the cut tables; plain: room for split tasks) */
 } dto_job_info;
 
 typedef struct dto_job dto_job;

@@ -114,3 +114,23 @@ def test_first_launches_on_two_streams(dto, gpu, n):
         assert all(torch.equal(o, w) for o in outs)
         job.close()
     want.close()
+
+
+def test_device_bytes_counts_every_allocation(dto, gpu):
+    """The footprint a job reports: the tables alone before the upload, then
+    what the upload and the first launch of each mode allocate."""
+    n = 36000
+    job = dto.Job.from_lists(*_lists(n), defer_upload=True)
+    deferred = job.device_bytes
+    seen = [deferred]
+    for call in (lambda: job.process_threshold_pairs(), lambda: job.optimize(mode="plain"), lambda: job.optimize()):
+        call()
+        seen.append(job.device_bytes)
+    assert seen == sorted(seen) and seen[1] > deferred + 2 * n * 1024  # staging: 1,024 slots of 16-bit rows
+    assert seen[2] > seen[1]
+    t1, t2 = job.n_thresholds1, job.n_thresholds2
+    assert seen[3] - seen[2] > 14 * t1 * t2 * 2  # 14 levels of 16-bit counts
+    job.set_thresholds(np.arange(1, 40), np.arange(1, 40))
+    assert job.device_bytes < seen[2]
+    job.close()
+    assert job.device_bytes > 0
