@@ -233,13 +233,11 @@ int upload_job(dto_job *j) {
     j->ws_bytes = ws_bytes;
     if (!j->ws_ev) HIP_TRY(hipEventCreateWithFlags(&j->ws_ev, hipEventDisableTiming));
   }
-  /* after the tables: the error word, the records of a small run and one
-   * pair of index arrays, so that calls need no allocation of their own and
-   * one copy brings the error word and the records back */
+  /* after the tables: the room of a small call, which then needs no
+   * allocation of its own; one copy brings its error word and records back */
   const size_t tables = j->image.size();
   j->image.resize(tables + kErrBytes, 0);
-  const size_t own_bytes = j->image.size() + kCallRecords * sizeof(dto_record) +
-                           ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t);
+  const size_t own_bytes = tables + kRoomIdx + ((size_t)j->dev.N1 + j->dev.N2) * sizeof(uint32_t);
   HIP_TRY(j->alloc(&j->arena, own_bytes));
   j->own_bytes = own_bytes;
   HIP_TRY(hipMemcpy(j->arena, j->image.data(), j->image.size(), hipMemcpyHostToDevice));
@@ -270,25 +268,27 @@ static uint32_t perm_grid(const dto_job *j, const LdsLayout &lo, uint64_t n_perm
 }
 
 /* lead = 1: the unpermuted task runs first, in the same launch, into record 0
- * (screened mode with drawn permutations only). */
+ * (screened mode with drawn permutations only).  part: see launch_plain. */
 static int launch_perms(dto_job *j, uint32_t mode, bool expl, const uint32_t *d1, const uint32_t *d2, uint64_t n_perm,
                         uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted, dto_record *d_out,
-                        hipStream_t st, uint32_t lead = 0) {
+                        hipStream_t st, uint32_t lead = 0, BestKey *part = nullptr) {
   if (n_perm + lead == 0) return DTO_OK;
   if (n_perm >= (1ull << 32) - 65536ull) return fail(DTO_ERR_TOO_LARGE, "too many permutations in one launch");
   hipError_t e;
   if (mode == DTO_MODE_PLAIN) {
     /* at most one workgroup per staging slot */
     const uint32_t g = perm_grid(j, j->lo_plain, ~0ull, 4);
-    e = launch_plain(j, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out);
+    e = launch_plain(j, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, d_out, part);
   } else if (mode == DTO_MODE_SCREENED) {
     const uint32_t *cut = nullptr;
     int rc = cut_tables(j, st, &cut);
     if (rc) return rc;
     if (!cut) {
       /* no memory for the tables: the plain kernels give the same records */
-      if (lead && (rc = launch_perms(j, DTO_MODE_PLAIN, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_out, st))) return rc;
-      return launch_perms(j, DTO_MODE_PLAIN, expl, d1, d2, n_perm, base, seed, job_id, permuted, d_out + lead, st);
+      if (lead && (rc = launch_perms(j, DTO_MODE_PLAIN, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_out, st, 0, part)))
+        return rc;
+      return launch_perms(j, DTO_MODE_PLAIN, expl, d1, d2, n_perm, base, seed, job_id, permuted, d_out + lead, st, 0,
+                          part);
     }
     const uint32_t g = perm_grid(j, j->lo_cut, n_perm + lead, j->cut_sh.nt == 512 ? 4 : 2);
     e = launch_cut(j, cut, expl, g, st, d1, d2, n_perm, base, seed, job_id, permuted, lead, d_out);
@@ -319,14 +319,15 @@ struct DevBuf {
 };
 
 /* Device room for one call's records (and, for a single explicit pair, its
- * index arrays): the job's own where it is free and large enough, else
- * allocated for the call. */
+ * index arrays; for plain launches, their partial results): the job's own
+ * where it is free and large enough, else allocated for the call. */
 struct CallRoom {
   dto_job *j;
   std::unique_lock<std::mutex> own;
   DevBuf tmp;
   dto_record *rec = nullptr;
   uint32_t *idx = nullptr;
+  BestKey *part = nullptr;
   size_t records = 0;
   explicit CallRoom(dto_job *job) : j(job) {}
   int open(size_t n, bool with_idx) {
@@ -335,8 +336,10 @@ struct CallRoom {
     if (j->arena && n <= kCallRecords) {
       own = std::unique_lock<std::mutex>(j->call_mu, std::try_to_lock);
       if (own.owns_lock()) {
-        rec = (dto_record *)((unsigned char *)j->d_err + kErrBytes);
-        idx = (uint32_t *)(rec + kCallRecords);
+        unsigned char *const room = (unsigned char *)j->d_err;
+        rec = (dto_record *)(room + kErrBytes);
+        part = (BestKey *)(room + kRoomPart);
+        idx = (uint32_t *)(room + kRoomIdx);
         return DTO_OK;
       }
     }
@@ -684,7 +687,7 @@ int dto_optimize(dto_job *job, const uint32_t *idx1, const uint32_t *idx2, uint3
     HIP_TRY(hipMemcpy(d2, idx2, n2 * 4, hipMemcpyHostToDevice));
   }
   int32_t permuted = (idx1 || idx2) ? 1 : 0;
-  if ((rc = launch_perms(job, mode, true, d1, d2, 1, 0, 0, 0, permuted, room.rec, 0))) return rc;
+  if ((rc = launch_perms(job, mode, true, d1, d2, 1, 0, 0, 0, permuted, room.rec, 0, 0, room.part))) return rc;
   std::vector<unsigned char> buf;
   const dto_record *rec = nullptr;
   if ((rc = room.fetch(buf, &rec))) return rc;
@@ -746,7 +749,7 @@ int dto_run(dto_job *job, uint64_t n_perm, uint64_t seed, const uint32_t *idx1, 
   /* task 0: unpermuted (main.rs:122-125); with drawn permutations it joins
    * their launch, where it costs no workgroup's latency of its own */
   const uint32_t lead = mode == DTO_MODE_SCREENED && n_perm && !idx1 ? 1 : 0;
-  if (!lead && (rc = launch_perms(job, mode, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_rec, 0))) return rc;
+  if (!lead && (rc = launch_perms(job, mode, true, nullptr, nullptr, 1, 0, 0, 0, 0, d_rec, 0, 0, room.part))) return rc;
   if (n_perm) {
     if (idx1) {
       /* explicit permutations, streamed in chunks of at most ~512 MiB */
@@ -759,11 +762,12 @@ int dto_run(dto_job *job, uint64_t n_perm, uint64_t seed, const uint32_t *idx1, 
         uint64_t c = std::min(chunk, n_perm - p0);
         HIP_TRY(hipMemcpy(d1, idx1 + p0 * n1, c * n1 * 4, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(d2, idx2 + p0 * n2, c * n2 * 4, hipMemcpyHostToDevice));
-        if ((rc = launch_perms(job, mode, true, d1, d2, c, p0, seed, 0, 1, d_rec + 1 + p0, 0))) return rc;
+        if ((rc = launch_perms(job, mode, true, d1, d2, c, p0, seed, 0, 1, d_rec + 1 + p0, 0, 0, room.part))) return rc;
         HIP_TRY(hipDeviceSynchronize());
       }
     } else {
-      if ((rc = launch_perms(job, mode, false, nullptr, nullptr, n_perm, 0, seed, 0, 1, d_rec + 1 - lead, 0, lead)))
+      if ((rc = launch_perms(job, mode, false, nullptr, nullptr, n_perm, 0, seed, 0, 1, d_rec + 1 - lead, 0, lead,
+                             room.part)))
         return rc;
     }
   }

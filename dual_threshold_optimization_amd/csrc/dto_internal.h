@@ -66,9 +66,17 @@ struct LaunchSlots {
   }
   uint32_t take(hipStream_t st) { return take(stream_capturing(st)); }
 };
-/* A resident job's room for small calls (upload_job): bytes of the error
- * word's block, and records after it (a run of 1,000 permutations). */
+/* Plain launches of at most kSplitTasks tasks split each over several
+ * workgroups, kSplitItems in all (two for each CU), whose partial results go
+ * to a buffer. */
+constexpr uint32_t kSplitTasks = 256, kSplitItems = 512;
+/* A resident job's room for small calls (upload_job), after its tables: the
+ * error word's block, records (a run of 1,000 permutations), the partial
+ * results of one plain launch, and one pair of index arrays. */
 constexpr size_t kErrBytes = 256, kCallRecords = 1025;
+constexpr size_t kRoomPart = kErrBytes + kCallRecords * sizeof(dto_record);
+constexpr size_t kRoomIdx = kRoomPart + kSplitItems * sizeof(dto::BestKey);
+static_assert(kRoomPart % alignof(dto::BestKey) == 0, "partial results follow the records");
 
 /* Byte offsets of a job's tables inside its device arena. */
 struct ArenaOffsets {
@@ -173,9 +181,11 @@ int cut_tables(dto_job *j, hipStream_t st, const uint32_t **out);
 hipError_t launch_cut(dto_job *j, const uint32_t *cut, bool expl, uint32_t grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
                       uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted, uint32_t lead,
                       dto_record *out);
+/* part: the caller's room for the partial results (kSplitItems), or NULL for
+ * a slot of the job's own buffer. */
 hipError_t launch_plain(dto_job *j, bool expl, uint32_t max_grid, hipStream_t st, const uint32_t *i1,
                         const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id,
-                        int32_t permuted, dto_record *out);
+                        int32_t permuted, dto_record *out, BestKey *part);
 struct BatchJob;
 struct WorkItem;
 hipError_t launch_batch_cut(const CutShape &sh, uint32_t grid, hipStream_t st, const BatchJob *jobs,

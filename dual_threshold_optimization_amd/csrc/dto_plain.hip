@@ -12,13 +12,9 @@
 
 using namespace dto;
 
-/* Launches of at most kSplitTasks tasks split each over several workgroups,
- * kSplitItems in all (two for each CU); their partial results go to the
- * launch's slot of a buffer that the job keeps from its first plain launch on. */
-constexpr uint32_t kSplitTasks = 256, kSplitItems = 512;
-
-/* The launch's slot of the partial buffer, or NULL where there is no memory
- * for it (the launch is then not split). */
+/* The launch's slot of the buffer of partial results that the job keeps from
+ * its first split launch on, or NULL where there is no memory for it (the
+ * launch is then not split). */
 static BestKey *partial_slot(dto_job *j, uint32_t slot) {
   std::lock_guard<std::mutex> g(j->cut_mu);
   if (!j->partial) {
@@ -36,17 +32,17 @@ static BestKey *partial_slot(dto_job *j, uint32_t slot) {
 template <bool E, bool PL>
 static hipError_t launch_t(dto_job *j, uint32_t max_grid, hipStream_t st, const uint32_t *i1, const uint32_t *i2,
                            uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id, int32_t permuted,
-                           dto_record *out) {
+                           dto_record *out, BestKey *part) {
   auto kern = k_plain<kNT, E, PL>;
   const LdsLayout &lo = j->lo_plain;
   (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lo.total);
   const uint32_t slot = j->slots.take(st);
   uint32_t *ctr = j->d_ctr + slot;
   uint32_t parts = 1;
-  BestKey *partial = nullptr;
+  BestKey *partial = part;
   if (n_perm <= kSplitTasks) {
     parts = std::min<uint32_t>(kSplitItems / (uint32_t)n_perm, (j->dev.T1 + kNT / 64 - 1) / (kNT / 64));
-    if (parts > 1 && !(partial = partial_slot(j, slot))) parts = 1;
+    if (parts > 1 && !partial && !(partial = partial_slot(j, slot))) parts = 1;
   }
   const uint32_t grid = (uint32_t)std::min<uint64_t>(n_perm * parts, max_grid);
   StagingOrder order(j, lo, st);
@@ -61,12 +57,12 @@ static hipError_t launch_t(dto_job *j, uint32_t max_grid, hipStream_t st, const 
 
 hipError_t dto::launch_plain(dto_job *j, bool expl, uint32_t max_grid, hipStream_t st, const uint32_t *i1,
                              const uint32_t *i2, uint64_t n_perm, uint64_t base, uint64_t seed, uint32_t job_id,
-                             int32_t permuted, dto_record *out) {
+                             int32_t permuted, dto_record *out, BestKey *part) {
   if (j->lo_plain.pairs_in_lds)
-    return expl ? launch_t<true, true>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out)
-                : launch_t<false, true>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
-  return expl ? launch_t<true, false>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out)
-              : launch_t<false, false>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out);
+    return expl ? launch_t<true, true>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out, part)
+                : launch_t<false, true>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out, part);
+  return expl ? launch_t<true, false>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out, part)
+              : launch_t<false, false>(j, max_grid, st, i1, i2, n_perm, base, seed, job_id, permuted, out, part);
 }
 
 /* The debug grid of one permutation on a stream: overlap counts into kcnt

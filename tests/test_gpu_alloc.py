@@ -81,17 +81,33 @@ def test_batch_without_cut_tables(dto, gpu, n):
 
 @pytest.mark.parametrize("nth", [2, 3])
 def test_creation_needs_no_cut_tables(dto, gpu, nth):
-    """An upload at this size makes one allocation.  The next are the split
-    plain launches' partial results and, from the first screened call on, the
-    cut tables: calls that can do without them do."""
+    """An upload at this size makes one allocation.  The next are, from the
+    first screened call on, the cut tables and, from the first asynchronous
+    plain launch on, the partial results: calls that can do without them do."""
+    import torch
     job = dto.Job.from_lists(*_lists(3000), defer_upload=True)
     _fail_alloc(dto, job, nth)
     want = dto.Job.from_lists(*_lists(3000))
     assert job.optimize(mode="plain") == want.optimize(mode="plain")
     assert job.process_threshold_pairs().tobytes() == want.process_threshold_pairs().tobytes()
     assert job.optimize() == want.optimize()
+    rec = torch.zeros(2, 5 * 72, dtype=torch.uint8, device="cuda:0")
+    for j, r in zip((job, want), rec):
+        j.run_device(5, r.data_ptr(), seed=2, mode="plain")
+    torch.cuda.synchronize()
+    assert torch.equal(rec[0], rec[1])
     job.close()
     want.close()
+
+
+def test_plain_call_allocates_nothing(dto, gpu):
+    """A plain call that fits the job's call room needs no memory of its own."""
+    job = dto.Job.from_lists(*_lists(200))
+    held = job.device_bytes
+    job.optimize(mode="plain")
+    job.run(20, seed=1, mode="plain")
+    assert job.device_bytes == held
+    job.close()
 
 
 @pytest.mark.parametrize("n", [900, 20000])
@@ -119,13 +135,17 @@ def test_first_launches_on_two_streams(dto, gpu, n):
 def test_device_bytes_counts_every_allocation(dto, gpu):
     """The footprint a job reports: the tables alone before the upload, then
     what the upload and the first launch of each mode allocate."""
+    import torch
     n = 36000
     job = dto.Job.from_lists(*_lists(n), defer_upload=True)
     deferred = job.device_bytes
     seen = [deferred]
-    for call in (lambda: job.process_threshold_pairs(), lambda: job.optimize(mode="plain"), lambda: job.optimize()):
+    out = torch.zeros(72, dtype=torch.uint8, device="cuda:0")
+    for call in (lambda: job.process_threshold_pairs(), lambda: job.run_device(1, out.data_ptr(), mode="plain"),
+                 lambda: job.optimize()):
         call()
         seen.append(job.device_bytes)
+    torch.cuda.synchronize()
     assert seen == sorted(seen) and seen[1] > deferred + 2 * n * 1024  # staging: 1,024 slots of 16-bit rows
     assert seen[2] > seen[1]
     t1, t2 = job.n_thresholds1, job.n_thresholds2
