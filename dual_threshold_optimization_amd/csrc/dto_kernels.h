@@ -1220,11 +1220,9 @@ __device__ __forceinline__ ZeroKey class1_best(const DevJob &J, const LdsLayout 
 /* One permutation: overlap grid -> best cell.  Returns the best key in
  * thread 0 (others: undefined).  Rows are interleaved over the waves: every
  * wave adds every row's pairs to its own running column counts, and scans
- * the rows i with i % W == w.  ZCM, the screen's k > K test (cells with an
- * empty tail): 1 in, 0 left out (the job cannot have such cells,
- * DevJob.kle), 2 chosen by J.kle at run time (the batch kernel, whose jobs
- * differ). */
-template <int NT, bool EXPLICIT, bool HLDS, bool PL, bool REGCOLS, bool NBL = true, int ZCM = 2>
+ * the rows i with i % W == w.  The screen's k > K test (cells with an empty
+ * tail) is left out for jobs that cannot have such cells (DevJob.kle). */
+template <int NT, bool EXPLICIT, bool HLDS, bool PL, bool REGCOLS, bool NBL = true>
 __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayout &Lo, const Lds &S, const uint32_t *i1,
                                  const uint32_t *i2, const Shuffle &s1, const Shuffle &s2, int *err,
                                  WaveStats &st, uint16_t *gpairs) {
@@ -1320,7 +1318,7 @@ __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayou
       if (REGCOLS) run = wave_excl_scan(tot);
       uint32_t kk[kSegCells], nn4[kSegCells];
       float xx[kSegCells];
-      if (ZCM == 2 ? J.kle != 0u : ZCM == 0)
+      if (J.kle)
         segment_fast<HLDS, REGCOLS, false>(J, S, Hb, wv, nseg, wbeg + t0, run, K, NK4, A, cr, kk, nn4, xx);
       else
         segment_fast<HLDS, REGCOLS, true>(J, S, Hb, wv, nseg, wbeg + t0, run, K, NK4, A, cr, kk, nn4, xx);
@@ -1480,7 +1478,7 @@ __device__ __forceinline__ BestKey optimize_perm(const DevJob &J, const LdsLayou
         if (REGCOLS) run = wave_excl_scan(tot);
         uint32_t kk[kSegCells], nn4[kSegCells];
         float xx[kSegCells];
-        if (ZCM == 2 ? J.kle != 0u : ZCM == 0)
+        if (J.kle)
           segment_fast<HLDS, REGCOLS, false>(J, S, Hb, wv, nseg, wbeg + t0, run, K, NK4, A, cr, kk, nn4, xx);
         else
           segment_fast<HLDS, REGCOLS, true>(J, S, Hb, wv, nseg, wbeg + t0, run, K, NK4, A, cr, kk, nn4, xx);
