@@ -145,6 +145,7 @@ INTERNAL = {
     "dto_internal_stats": (_int, [_vp, _P(_u64), _int]),
     "dto_internal_launch_slots": (_int, [_P(_i32), _u32, _P(_u32)]),
     "dto_internal_fail_alloc": (_int, [_vp, _u32]),
+    "dto_internal_cut_shape": (_int, [_vp, _P(_i32), _P(_i32)]),
     "dto_internal_philox": (_int, [_P(_u32), _P(_u32), _P(_u32)]),
     "dto_internal_read_ranked_csv": (_int, [_cp, _vp, _u64, _P(_u64), _P(_u32), _u64, _P(_u64)]),
     "dto_internal_read_feature_lines": (_int, [_cp, _vp, _u64, _P(_u64), _P(_u64)]),

@@ -541,6 +541,14 @@ int dto_internal_launch_slots(const int32_t *captured, uint32_t n, uint32_t *out
   return DTO_OK;
 }
 
+/* test hook (not in dto.h): threads and build of the job's screened launches */
+int dto_internal_cut_shape(const dto_job *job, int32_t *nt, int32_t *build) {
+  if (!job || !nt || !build) return fail(DTO_ERR_INVALID_ARGUMENT, "null pointer");
+  *nt = job->cut_sh.nt;
+  *build = job->cut_sh.build;
+  return DTO_OK;
+}
+
 /* test hook (not in dto.h): the n-th device allocation of the job from now on
  * fails (0: none does) */
 int dto_internal_fail_alloc(dto_job *job, uint32_t n) {

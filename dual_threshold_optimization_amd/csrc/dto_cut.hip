@@ -53,7 +53,9 @@ bool dto::cut_layout(const HostJob &h, int W, int build, LdsLayout *out) {
 
 /* One shape for a set of jobs: 512-thread workgroups where two or more fit a
  * CU (the waves of one hide the barriers of another), else 1,024 threads, so
- * that a CU holds 16 waves either way; the first build that every job fits. */
+ * that a CU holds 16 waves either way; the first build that every job fits.
+ * Where 16 waves' column counts do not fit beside the lists or the thresholds
+ * (reference thresholds: above 49,800 entries), 512 threads, 8 waves a CU. */
 int dto::cut_shape(const HostJob *const *jobs, size_t n, size_t lim, CutShape *out) {
   const struct {
     int nt, build;

@@ -44,9 +44,9 @@ def test_column_segments(dto, gpu, t2, kind):
     job.close()
 
 
-# 512 threads up to about 13,700 entries; 1,024 with pairs in registers to about
-# 21,000, in LDS to about 31,000, in global memory above; shuffle domains of
-# 16,384 and 32,768 elements are the most that the registers of either hold
+# with the 60 thresholds set here: 512 threads with pairs in registers to 15,248
+# entries, in LDS to 19,280, 1,024 with pairs in registers to 31,136, in LDS to
+# 39,264, in global memory above (the edges themselves: test_gpu_shapes.py)
 @pytest.mark.parametrize("n", [1, 2, 5, 63, 65, 13500, 13900, 16300, 16500, 20900, 23500, 32700, 33100, 41000])
 @pytest.mark.parametrize("explicit", [False, True])
 def test_shapes(dto, gpu, n, explicit):
