@@ -519,10 +519,11 @@ int dto_internal_shuffle_device(uint64_t seed, uint32_t job, uint32_t perm, uint
 }
 
 /* work counters of a job's screened launches (test / profiling hook, not in
- * dto.h), 16 values: exact cells, exact terms, rescanned rows, cycles of the
- * build / forward / reverse / tier-1 flush / exact phases, tier-1 pushes,
- * tier-2 survivors, tier-1 flushes, first-bound gap (milli-nats), cells past
- * the reverse sweep's first-term test */
+ * dto.h), 16 values: exact cells, exact terms, passes, cycles of the build /
+ * column counts / sweep / list flushes / what follows the sweep, cells past
+ * the first-term test, tier-2 survivors, tier-2 flushes, 0, listed cells; in a
+ * server's slices what the first-term screen counts in their places
+ * (WaveStats) */
 int dto_internal_stats(dto_job *job, uint64_t *out, int reset) {
   if (!job || !out) return fail(DTO_ERR_INVALID_ARGUMENT, "null pointer");
   if (!DTO_STATS) return fail(DTO_ERR_INVALID_ARGUMENT, "the library was built without DTO_STATS (make STATS=1)");

@@ -4,9 +4,11 @@
  * The reference runs one job per process and spreads its permutations over
  * std::thread chunks (src/run/single_node.rs:83-137) or MPI ranks
  * (src/run/multi_node.rs:47-162).  Here many jobs of uneven size share one
- * persistent kernel (k_batch): every workgroup pulls (job, task range) items
- * from a device queue until it is empty.  A batch's launch sequence (queue
- * reset + persistent kernel) is captured once in a hipGraph and replayed.
+ * persistent kernel: every workgroup pulls (job, task range) items from a
+ * device queue until it is empty.  Batches run k_batch_cut (dto_cut.h), a
+ * server's slices k_batch (dto_kernels.h), which needs no cut tables.  A
+ * batch's launch sequence (queue reset + persistent kernel) is captured once
+ * in a hipGraph and replayed.
  *
  * The server does continuous batching: requests are admitted, oldest first,
  * while their tables and records fit a device pool of hbm_budget_bytes (one

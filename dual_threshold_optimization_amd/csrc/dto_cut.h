@@ -66,11 +66,14 @@ __device__ __forceinline__ double log_term(const DevJob &J, uint32_t K, uint32_t
  * lane + u.  A cell is dropped when k <= its cut.  One thread per cell.  For
  * the low levels the cut is the largest k found with P(X = k) alone above the
  * level.  From there it adds terms downwards in FP32: at every k the sum is a
- * lower bound of P(X >= k) up to its rounding (each term's ratio has a
- * relative error below 4 * 2^-24, and above populations of 2^24 the counts'
- * own rounding adds under 0.6 % at the longest accepted lists), so P(X >= k)
- * > e^l is certain once the sum exceeds 1.01 e^l, and for every smaller k
- * too.  A tail that never gets there keeps the cut max(0, K + n - N), the
+ * lower bound of P(X >= k) up to its rounding: each term's ratio has a
+ * relative error of up to 6 * 2^-24 (four roundings and a reciprocal of 1
+ * ulp), and fewer than 1,000 steps lead from the low levels to 1.2 standard
+ * deviations (at most 99) below the mean, where the sum exceeds the highest
+ * level: under 0.04 %.  Above populations of 2^24, where subtracting 1 from a
+ * count is rounded too, the deviation is at most 16, and fewer than 200 steps
+ * add under 0.12 %.  So P(X >= k) > e^l is certain once the sum exceeds 1.01
+ * e^l, and for every smaller k too.  A tail that never gets there keeps the cut max(0, K + n - N), the
  * largest k with P(X >= k) = 1, which is also level 0's.  Columns past T2 get
  * 0xFFFF: never listed.  89 us at 599 x 599 cells and 14 levels; adding every
  * term from the lowest level up took 245 us. */

@@ -67,8 +67,9 @@ struct LaunchSlots {
   uint32_t take(hipStream_t st) { return take(stream_capturing(st)); }
 };
 /* Plain launches of at most kSplitTasks tasks split each over several
- * workgroups, kSplitItems in all (two for each CU), whose partial results go
- * to a buffer. */
+ * workgroups, kSplitItems in all, whose partial results go to a buffer of that
+ * size: two for each of this GPU's 256 CUs (a task alone fills it; 257 tasks
+ * and more occupy it as they are). */
 constexpr uint32_t kSplitTasks = 256, kSplitItems = 512;
 /* A resident job's room for small calls (upload_job), after its tables: the
  * error word's block, records (a run of 1,000 permutations), the partial

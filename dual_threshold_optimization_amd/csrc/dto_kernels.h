@@ -8,8 +8,9 @@
  * One workgroup owns one permutation at a time.  This file holds what the
  * kernels share (the build of a permutation's row-sorted pairs, the exact
  * and bracket tiers, the tie-break) and the first-term screen of serving
- * slices; dto_cut.h holds the screened kernels of jobs with cut tables,
- * dto_plain.h the plain mode and the debug grid.
+ * slices and of batches whose jobs found no memory for cut tables; dto_cut.h
+ * holds the screened kernels of jobs with cut tables, dto_plain.h the plain
+ * mode and the debug grid.
  *   A  scatter: list1 feature m takes the bin of the position it lands on,
  *      nb[idx1[k]] = bin1[k]                                  (LDS, u16)
  *   B  pairs: list2 position e holds entry q = idx2[e]; its list1 partner's
@@ -682,11 +683,15 @@ __device__ __forceinline__ double first_exponent(const DevJob &J, uint32_t K, ui
 }
 
 struct WaveStats {
-  uint32_t cells, terms, rows;
-  uint64_t cyc[5]; /* build, forward sweep, reverse sweep, tier-2 brackets (flush_candidates), exact */
+  uint32_t cells, terms;
+  uint32_t rows; /* rows rescanned by the reverse sweep; optimize_cut: passes */
+  /* build, forward sweep, reverse sweep, tier-2 brackets (flush_candidates),
+   * exact; optimize_cut: build, column counts, sweep (flush_cut in it
+   * included), flush_cut, what follows the sweep */
+  uint64_t cyc[5];
   uint32_t push1, push2, flushes; /* tier-1 survivors, tier-2 survivors, flush_candidates calls */
-  uint32_t gap;                    /* sum of (first upper bound - log of the minimum), milli-nats */
-  uint32_t cheap;                  /* cells passing the first-term test of the reverse sweep (per lane) */
+  uint32_t gap;   /* sum of (first upper bound - log of the minimum), milli-nats; optimize_cut: 0 */
+  uint32_t cheap; /* cells passing the reverse sweep's first-term test (per lane); optimize_cut: listed cells */
 };
 
 __device__ __forceinline__ uint64_t cycles() {

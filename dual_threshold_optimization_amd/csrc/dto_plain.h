@@ -177,7 +177,7 @@ __global__ __launch_bounds__(NT) void k_grid_counts(DevJob J, LdsLayout Lo, cons
 }
 
 /* Exact p-value of every cell from the count grid.  A wave's 64 records are
- * put together in LDS and stored as consecutive 16-byte words (72-byte
+ * put together in LDS and stored as consecutive 8-byte words (72-byte
  * records written lane by lane touch every line 18 times). */
 static __global__ __launch_bounds__(256) void k_grid_pvalues(DevJob J, const uint32_t *__restrict__ kin,
                                                              int32_t permuted, dto_record *__restrict__ out) {

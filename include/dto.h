@@ -216,8 +216,9 @@ int dto_batch_launch(dto_batch *b, void *stream);
 /* Copy results: one dto_result per job. */
 int dto_batch_results(dto_batch *b, dto_result *results);
 void dto_batch_destroy(dto_batch *b);
-/* Autotuner: times the candidate launch shapes on this batch and keeps the
- * fastest; returns the chosen waves-per-workgroup through *waves. */
+/* Autotuner: times the candidate queues (1, 4 and 16 tasks per work item) on
+ * this batch and keeps the fastest; returns the waves per workgroup, which the
+ * sizes of the jobs decide (8 or 16), through *waves. */
 int dto_batch_autotune(dto_batch *b, int *waves);
 
 /* ---- serving (continuous batching) --------------------------------------- */
